@@ -148,6 +148,7 @@ struct route_cache {
   uint16_t first_child[kMaxNodes];  // slot of its first child, or kNoChild
   uint32_t count;                   // slots routed through (internal node images)
   uint32_t stop;                    // build: the last level has been reached
+  uint32_t leaves;                  // build: the level being read holds leaves
 };
 
 template <int NW, bool VER>
@@ -778,18 +779,22 @@ struct tree_view : tree_ptrs {
   }
 
   // Block-wide (every thread of the workgroup calls it, before any early
-  // return; blockDim.x >= 64): copies the top levels into `rc`. The cache
-  // stays empty (routing starts at the root) while fewer than `min_nodes`
-  // nodes have been handed out.
+  // return; blockDim.x a multiple of 64): copies the top levels into `rc`.
+  // The cache stays empty (routing starts at the root) while fewer than
+  // `min_nodes` nodes have been handed out (~0: always).
+  // One load round and one scan per level, every part of it spread over the
+  // workgroup: NW lanes load a node and count its entries with a ballot, wave
+  // 0 turns the counts into child slots, and all threads file the children.
   template <class RC>
   MVBT_DEV void build_route_cache(RC& rc, unsigned long long min_nodes = 0) const {
     using rc_t = RC;
     const uint32_t tid = threadIdx.x, nthreads = blockDim.x;
     if (tid == 0) {
-      const bool use = min_nodes == 0 || ld_coherent((const uint64_t*)&st->bump) >= min_nodes;
+      const bool use = min_nodes == 0 || (min_nodes != ~0ull && ld_coherent((const uint64_t*)&st->bump) >= min_nodes);
       rc.index[0] = root_;
       rc.count = use ? 1u : 0u;
       rc.stop = use ? 0u : 1u;
+      rc.leaves = 0;
     }
     __syncthreads();
     if (rc.stop) return;
@@ -798,23 +803,24 @@ struct tree_view : tree_ptrs {
     // the build stops (rc.stop) within kMaxNodes levels
     for (uint32_t level = 0; level < rc_t::kMaxNodes; ++level) {
       for (uint32_t w = tid; w < (e - b) * NW; w += nthreads) {
-        const uint32_t s = b + w / NW;
-        rc.img(s)[w % NW] = ld_coherent(at(rc.index[s]) + w % NW);
+        const uint32_t s = b + w / NW, l = w % NW;
+        const uint64_t v = ld_coherent(at(rc.index[s]) + l);
+        rc.img(s)[l] = v;
+        // leading entries only: an image read during a split may have gaps
+        // (bit kData is never set, so the complement has a lowest bit)
+        const uint64_t has = __builtin_amdgcn_ballot_w64(l < node_t::kData && lo32(v) != kEmpty) >> (tid & (64 - NW));
+        if (l == node_t::kMetaLane) {
+          rc.first_child[s] = (uint16_t)__builtin_ctzll(~(has & ((1ull << node_t::kData) - 1)));
+          if (hi32(v) & kLeafBit) rc.leaves = 1;
+        }
       }
       __syncthreads();
-      if (tid < 64) {  // wave 0: child counts, prefix sum, child slots
+      if (tid < 64) {  // wave 0: entry counts to child slots
         const uint32_t lane = tid;
         uint32_t next = e;
-        bool all_internal = true;
         for (uint32_t s0 = b; s0 < e; s0 += 64) {
           const uint32_t s = s0 + lane;
-          uint32_t cnt = 0;
-          bool internal = true;
-          if (s < e) {  // leading entries only: an image read during a split may have gaps
-            internal = !(hi32(rc.img(s)[NW - 1]) & kLeafBit);
-            while (cnt < node_t::kData && lo32(rc.img(s)[cnt]) != kEmpty) ++cnt;
-          }
-          all_internal = all_internal && __builtin_amdgcn_ballot_w64(!internal) == 0;
+          const uint32_t cnt = s < e ? rc.first_child[s] : 0u;
           uint32_t incl = cnt;  // inclusive scan over the wave
           for (uint32_t d = 1; d < 64; d <<= 1) {
             const uint32_t up = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((lane >= d ? lane - d : lane) << 2), (int)incl);
@@ -823,32 +829,30 @@ struct tree_view : tree_ptrs {
           if (s < e) rc.first_child[s] = (uint16_t)(next + incl - cnt);
           next += (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
         }
-        const bool fits = all_internal && next <= rc_t::kMaxNodes && next > e;
-        for (uint32_t s = b + lane; s < e; s += 64) {
-          if (!fits) {
-            rc.first_child[s] = rc_t::kNoChild;
-            continue;
-          }
-          const uint32_t fc = rc.first_child[s];
-          for (uint32_t l = 0; l < node_t::kData; ++l) {
-            const uint64_t pr = rc.img(s)[l];
-            if (lo32(pr) == kEmpty) break;
-            rc.index[fc + l] = hi32(pr);
-          }
-        }
+        const bool internal = rc.leaves == 0;
+        const bool fits = internal && next <= rc_t::kMaxNodes && next > e;
+        if (!fits)
+          for (uint32_t s = b + lane; s < e; s += 64) rc.first_child[s] = rc_t::kNoChild;
         if (lane == 0) {
           if (fits) {
             rc.count = next;
           } else {
             rc.stop = 1;
-            if (!all_internal) rc.count = b;  // a level with leaves is not routed through
+            if (!internal) rc.count = b;  // a level with leaves is not routed through
           }
         }
       }
       __syncthreads();
       if (rc.stop) break;
+      const uint32_t next = rc.count;
+      for (uint32_t w = tid; w < (e - b) * NW; w += nthreads) {
+        const uint32_t s = b + w / NW, l = w % NW;
+        const uint32_t fc = rc.first_child[s], end = s + 1 < e ? (uint32_t)rc.first_child[s + 1] : next;
+        if (fc + l < end) rc.index[fc + l] = hi32(rc.img(s)[l]);
+      }
+      __syncthreads();
       b = e;
-      e = rc.count;
+      e = next;
     }
   }
 
