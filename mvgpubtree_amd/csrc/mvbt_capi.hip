@@ -160,13 +160,48 @@ struct device_guard {
   }
 };
 
-uint32_t grid_for(const mvbt_tree* t, uint64_t n, uint32_t nw, int waves_per_cu, int block = kBlock) {
-  const uint64_t ops_per_block = (uint64_t)block;  // one op per lane per chunk
-  uint64_t need = (n + ops_per_block - 1) / ops_per_block;
-  uint64_t cap = (uint64_t)t->num_cus * (uint64_t)waves_per_cu * 64 / (uint64_t)block;
-  (void)nw;
-  if (need < 1) need = 1;
-  return (uint32_t)std::min<uint64_t>(need, std::max<uint64_t>(cap, 1));
+// Workgroups of a launch of n operations, `per` to a tile of `width` lanes,
+// at most waves_per_cu waves on each CU.
+uint32_t grid_for(const mvbt_tree* t, uint64_t n, uint32_t width, uint32_t per, int waves_per_cu, int block = kBlock) {
+  const uint64_t ops_per_block = (uint64_t)block / width * per;
+  const uint64_t need = (n + ops_per_block - 1) / ops_per_block;
+  const uint64_t cap = (uint64_t)t->num_cus * (uint64_t)waves_per_cu * 64 / (uint64_t)block;
+  return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(need, std::max<uint64_t>(cap, 1)));
+}
+
+// How a launch of n operations is divided over tiles of `width` lanes: one
+// operation a tile while that leaves tiles idle, then as few as keep `waves`
+// waves of every CU busy in one round, up to one per lane. A tile works
+// through its operations a few at a time, each a chain of dependent loads, so
+// with fewer to a tile a small launch waits for fewer chains: on MI355X (32
+// pairs per node) 64 finds took 39.2 us with 16 to a tile and 8.5 with one,
+// 1000 updates 82 and 21, 64K range queries 65 and 29 (4 to a tile).
+// The top levels are copied to LDS only where a tile then routes at least
+// kCachedFrom operations through them: the copy takes 5-7 us, and the walk it
+// shortens is read once. 128K finds (4 to a tile) 26.3 us without it and 30.1
+// with, 256K (8) 45.2 and 41.6.
+constexpr uint32_t kCachedFrom = 5;
+work_split split_for(const mvbt_tree* t, uint64_t n, uint32_t width, int waves) {
+  const uint64_t tiles = (uint64_t)t->num_cus * (uint64_t)waves * (64 / width);
+  work_split ws;
+  ws.per_tile = (uint32_t)std::min<uint64_t>(width, (n + tiles - 1) / tiles);
+  ws.cached = ws.per_tile >= kCachedFrom ? 1u : 0u;
+  return ws;
+}
+constexpr int kFindWaves = 32, kRangeWaves = 16;  // about what the kernels hold of each CU
+
+// The same for write and mixed launches: a power of two (so a chunk lies in
+// one aligned group of `width` operations, see superseded()), for 12 waves on
+// each CU while a tile takes one or two and the 16 the kernels hold from there
+// up: with few operations a tile, more tiles cost more on the words they all
+// update than they save (16K updates: 43.6 us at 2 to a tile, 36.8 at 4).
+work_split split_writes(const mvbt_tree* t, uint64_t n, uint32_t width) {
+  work_split ws;
+  ws.per_tile = 1;
+  while (ws.per_tile < width && n > (uint64_t)ws.per_tile * t->num_cus * (ws.per_tile < 4 ? 12 : 16) * (64 / width))
+    ws.per_tile *= 2;
+  ws.cached = ws.per_tile >= kCachedFrom ? 1u : 0u;
+  return ws;
 }
 
 template <int NW, bool VER>
@@ -179,11 +214,12 @@ struct impl {
   // Read launches with tiles narrower than the node (no writer runs).
   template <int T>
   static bool find_wide(mvbt_tree* t, const uint32_t* keys, uint32_t* vals, uint64_t n, uint32_t ts, hipStream_t s,
-                        uint32_t g) {
+                        const work_split& ws) {
     if constexpr (T < NW && NW / T <= 4) {
       if (t->read_tile == (uint32_t)T) {
+        const uint32_t g = grid_for(t, n, T, ws.per_tile, 32, kFindBlock);
         hipLaunchKernelGGL((find_wide_kernel<NW, VER, T>), dim3(g), dim3(kFindBlock), 0, s,
-                           t->template view<NW, VER>(), keys, vals, n, ts);
+                           t->template view<NW, VER>(), keys, vals, n, ts, ws);
         return true;
       }
     }
@@ -191,11 +227,12 @@ struct impl {
   }
   template <int T>
   static bool range_wide(mvbt_tree* t, const uint32_t* lo, const uint32_t* hi, uint64_t* out, uint32_t* counts,
-                         uint32_t L, uint64_t n, uint32_t ts, hipStream_t s, uint32_t g) {
+                         uint32_t L, uint64_t n, uint32_t ts, hipStream_t s, const work_split& ws) {
     if constexpr (T < NW && NW / T <= 4) {
       if (t->read_tile == (uint32_t)T) {
+        const uint32_t g = grid_for(t, n, T, ws.per_tile, 32);
         hipLaunchKernelGGL((range_wide_kernel<NW, VER, T>), dim3(g), dim3(kBlock), 0, s,
-                           t->template view<NW, VER>(), lo, hi, out, counts, L, n, ts);
+                           t->template view<NW, VER>(), lo, hi, out, counts, L, n, ts, ws);
         return true;
       }
     }
@@ -203,44 +240,49 @@ struct impl {
   }
   static mvbt_status find(mvbt_tree* t, const uint32_t* keys, uint32_t* vals, uint64_t n,
                           uint32_t ts, hipStream_t s, bool conc) {
-    uint32_t g = grid_for(t, n, NW, 32, kFindBlock);
-    if (!conc && (find_wide<16>(t, keys, vals, n, ts, s, g) || find_wide<32>(t, keys, vals, n, ts, s, g))) {
+    const uint32_t width = !conc && t->read_tile ? t->read_tile : NW;
+    const work_split ws = split_for(t, n, width, kFindWaves);
+    if (!conc && (find_wide<16>(t, keys, vals, n, ts, s, ws) || find_wide<32>(t, keys, vals, n, ts, s, ws))) {
       MVBT_HIP(hipGetLastError());
       return MVBT_OK;
     }
+    const uint32_t g = grid_for(t, n, NW, ws.per_tile, 32, kFindBlock);
     if (conc)
       hipLaunchKernelGGL((find_kernel<NW, VER, true>), dim3(g), dim3(kFindBlock), 0, s,
-                         t->template view<NW, VER>(), keys, vals, n, ts);
+                         t->template view<NW, VER>(), keys, vals, n, ts, ws);
     else
       hipLaunchKernelGGL((find_kernel<NW, VER, false>), dim3(g), dim3(kFindBlock), 0, s,
-                         t->template view<NW, VER>(), keys, vals, n, ts);
+                         t->template view<NW, VER>(), keys, vals, n, ts, ws);
     MVBT_HIP(hipGetLastError());
     return MVBT_OK;
   }
   static mvbt_status range(mvbt_tree* t, const uint32_t* lo, const uint32_t* hi, uint64_t* out,
                            uint32_t* counts, uint32_t L, uint64_t n, uint32_t ts, hipStream_t s,
                            bool conc) {
-    uint32_t g = grid_for(t, n, NW, 32);
-    if (!conc && (range_wide<16>(t, lo, hi, out, counts, L, n, ts, s, g) ||
-                  range_wide<32>(t, lo, hi, out, counts, L, n, ts, s, g))) {
+    const uint32_t width = !conc && t->read_tile ? t->read_tile : NW;
+    const work_split ws = split_for(t, n, width, kRangeWaves);
+    if (!conc && (range_wide<16>(t, lo, hi, out, counts, L, n, ts, s, ws) ||
+                  range_wide<32>(t, lo, hi, out, counts, L, n, ts, s, ws))) {
       MVBT_HIP(hipGetLastError());
       return MVBT_OK;
     }
+    const uint32_t g = grid_for(t, n, NW, ws.per_tile, 32);
     if (conc)
       hipLaunchKernelGGL((range_kernel<NW, VER, true>), dim3(g), dim3(kBlock), 0, s,
-                         t->template view<NW, VER>(), lo, hi, out, counts, L, n, ts);
+                         t->template view<NW, VER>(), lo, hi, out, counts, L, n, ts, ws);
     else
       hipLaunchKernelGGL((range_kernel<NW, VER, false>), dim3(g), dim3(kBlock), 0, s,
-                         t->template view<NW, VER>(), lo, hi, out, counts, L, n, ts);
+                         t->template view<NW, VER>(), lo, hi, out, counts, L, n, ts, ws);
     MVBT_HIP(hipGetLastError());
     return MVBT_OK;
   }
   template <int OP>
   static mvbt_status write(mvbt_tree* t, const uint32_t* keys, const uint32_t* vals, uint64_t n,
                            hipStream_t s) {
-    uint32_t g = grid_for(t, n, NW, 32);
+    const work_split ws = split_writes(t, n, NW);
+    const uint32_t g = grid_for(t, n, NW, ws.per_tile, 32);
     hipLaunchKernelGGL((write_kernel<NW, VER, OP>), dim3(g), dim3(kBlock), 0, s,
-                       t->template view<NW, VER>(), keys, vals, n);
+                       t->template view<NW, VER>(), keys, vals, n, ws);
     MVBT_HIP(hipGetLastError());
     return MVBT_OK;
   }
@@ -260,9 +302,10 @@ struct impl {
                            const uint32_t* rhi, uint64_t nr, uint32_t* fout, uint64_t* pairs, uint32_t* counts,
                            uint32_t L, hipStream_t s) {
     if (VER) hipLaunchKernelGGL(mixed_setup_kernel, dim3(1), dim3(64), 0, s, t->st);
-    uint32_t g = grid_for(t, nw + nr, NW, 32);
+    const work_split ws = split_writes(t, nw + nr, NW);
+    const uint32_t g = grid_for(t, nw + nr, NW, ws.per_tile, 32);
     hipLaunchKernelGGL((mixed_kernel<NW, VER, IR>), dim3(g), dim3(kBlock), 0, s, t->template view<NW, VER>(), wk, wv,
-                       nw, rlo, rhi, nr, fout, pairs, counts, L);
+                       nw, rlo, rhi, nr, fout, pairs, counts, L, ws);
     MVBT_HIP(hipGetLastError());
     return MVBT_OK;
   }

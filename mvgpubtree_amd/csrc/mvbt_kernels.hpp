@@ -18,14 +18,24 @@ constexpr int kFindBlock = 1024;
 constexpr uint32_t kFindCacheBytes = 72 * 1024;
 constexpr uint32_t kRangeCacheBytes = 16 * 1024;
 
+// How a launch divides its operations (chosen on the host, split_for).
+struct work_split {
+  uint32_t per_tile;  // consecutive operations a tile takes at a time
+  uint32_t cached;    // nonzero: workgroups copy the tree's top levels to LDS first
+};
+
+// `per` consecutive operations a chunk (1 .. W): the lanes from `per` on hold none.
 template <int W>
 struct chunking {
   uint64_t first, stride;
-  MVBT_DEV chunking() {
+  uint32_t per;
+  MVBT_DEV explicit chunking(uint32_t ops_per_tile = W) : per(ops_per_tile) {
     const uint64_t tiles_per_block = blockDim.x / W;
-    first = ((uint64_t)blockIdx.x * tiles_per_block + threadIdx.x / W) * W;
-    stride = (uint64_t)gridDim.x * tiles_per_block * W;
+    first = ((uint64_t)blockIdx.x * tiles_per_block + threadIdx.x / W) * per;
+    stride = (uint64_t)gridDim.x * tiles_per_block * per;
   }
+  // Whether lane `rank` of the chunk at `base` holds operation base + rank of n.
+  MVBT_DEV bool holds(uint64_t base, uint32_t rank, uint64_t n) const { return rank < per && base + rank < n; }
 };
 
 // Creates the root (internal, pivot 0 -> first leaf) and the first, empty leaf.
@@ -175,14 +185,15 @@ MVBT_DEV uint32_t route_reads(const tree_view<NW, VER>& tv, uint32_t key, bool g
 template <int NW, bool VER, bool CONC>
 __global__ void __launch_bounds__(kFindBlock) __attribute__((amdgpu_waves_per_eu(8)))
 find_kernel(tree_view<NW, VER> tv, const uint32_t* keys,
-                                                          uint32_t* values, uint64_t n, uint32_t ts) {
+                                                          uint32_t* values, uint64_t n, uint32_t ts,
+                                                          work_split ws) {
   tile<NW> t;
-  chunking<NW> c;
+  chunking<NW> c(ws.per_tile);
   __shared__ route_cache<NW, kFindCacheBytes> rc;
-  tv.build_route_cache(rc);
+  tv.build_route_cache(rc, ws.cached ? 0ull : ~0ull);
   for (uint64_t base = c.first; base < n; base += c.stride) {
     uint64_t i = base + t.rank();
-    bool active = i < n;
+    bool active = c.holds(base, t.rank(), n);
     uint32_t key = active ? keys[i] : 0u;
     uint32_t result = kEmpty;
     uint64_t q = t.ballot(active);
@@ -213,14 +224,14 @@ find_kernel(tree_view<NW, VER> tv, const uint32_t* keys,
 template <int NW, bool VER, bool CONC>
 __global__ void __launch_bounds__(256)
     range_kernel(tree_view<NW, VER> tv, const uint32_t* lower, const uint32_t* upper,
-                 uint64_t* out, uint32_t* counts, uint32_t L, uint64_t n, uint32_t ts) {
+                 uint64_t* out, uint32_t* counts, uint32_t L, uint64_t n, uint32_t ts, work_split ws) {
   tile<NW> t;
-  chunking<NW> c;
+  chunking<NW> c(ws.per_tile);
   __shared__ route_cache<NW, kRangeCacheBytes> rc;
-  tv.build_route_cache(rc);
+  tv.build_route_cache(rc, ws.cached ? 0ull : ~0ull);
   for (uint64_t base = c.first; base < n; base += c.stride) {
     uint64_t i = base + t.rank();
-    bool active = i < n;
+    bool active = c.holds(base, t.rank(), n);
     uint32_t lo = active ? lower[i] : 0u;
     uint32_t hi = active ? upper[i] : 0u;
     uint32_t result = 0;
@@ -275,15 +286,16 @@ __global__ void __launch_bounds__(256)
 
 template <int NW, bool VER, int T>
 __global__ void __launch_bounds__(kFindBlock) __attribute__((amdgpu_waves_per_eu(8)))
-find_wide_kernel(tree_view<NW, VER> tv, const uint32_t* keys, uint32_t* values, uint64_t n, uint32_t ts) {
+find_wide_kernel(tree_view<NW, VER> tv, const uint32_t* keys, uint32_t* values, uint64_t n, uint32_t ts,
+                 work_split ws) {
   using rc_t = route_cache<NW, kFindCacheBytes>;
   tile<T> t;
-  chunking<T> c;
+  chunking<T> c(ws.per_tile);
   __shared__ rc_t rc;
-  tv.build_route_cache(rc);
+  tv.build_route_cache(rc, ws.cached ? 0ull : ~0ull);
   for (uint64_t base = c.first; base < n; base += c.stride) {
     const uint64_t i = base + t.rank();
-    const bool active = i < n;
+    const bool active = c.holds(base, t.rank(), n);
     const uint32_t key = active ? keys[i] : 0u;
     const uint32_t result =
         read_chunk_wide<T, false, false, kWideFindGroup<NW / T>>(tv, key, 0u, ts, nullptr, 0u, t.ballot(active), t, &rc);
@@ -294,15 +306,15 @@ find_wide_kernel(tree_view<NW, VER> tv, const uint32_t* keys, uint32_t* values, 
 template <int NW, bool VER, int T>
 __global__ void __launch_bounds__(256)
     range_wide_kernel(tree_view<NW, VER> tv, const uint32_t* lower, const uint32_t* upper, uint64_t* out,
-                      uint32_t* counts, uint32_t L, uint64_t n, uint32_t ts) {
+                      uint32_t* counts, uint32_t L, uint64_t n, uint32_t ts, work_split ws) {
   using rc_t = route_cache<NW, kRangeCacheBytes>;
   tile<T> t;
-  chunking<T> c;
+  chunking<T> c(ws.per_tile);
   __shared__ rc_t rc;
-  tv.build_route_cache(rc);
+  tv.build_route_cache(rc, ws.cached ? 0ull : ~0ull);
   for (uint64_t base = c.first; base < n; base += c.stride) {
     const uint64_t i = base + t.rank();
-    const bool active = i < n;
+    const bool active = c.holds(base, t.rank(), n);
     const uint32_t lo = active ? lower[i] : 0u;
     const uint32_t hi = active ? upper[i] : 0u;
     const uint32_t result = read_chunk_wide<T, true, false, kWideRangeGroup<NW / T>>(
@@ -312,11 +324,49 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// Inserts of a chunk of fewer than NW operations that a later one of the same
+// aligned group of NW operations supersedes (the same key): a mask over the
+// chunk's lanes. A tile that takes all NW applies them in order, the last one
+// winning; divided over several tiles they would race, so the earlier ones
+// are dropped. `per` divides NW: the chunk at `base` lies in one group.
+template <int NW>
+MVBT_DEV uint64_t superseded(const uint32_t* keys, uint64_t base, uint64_t n, uint32_t per, const tile<NW>& t) {
+  const uint64_t group = base & ~(uint64_t)(NW - 1);
+  const uint32_t r = t.rank(), first = (uint32_t)(base - group);
+  const uint32_t k = group + r < n ? keys[group + r] : 0u;
+  uint64_t drop = 0;
+  for (uint32_t j = 0; j < per && base + j < n; ++j) {
+    const uint32_t kj = t.shfl(k, first + j);
+    if (t.ballot(k == kj && r > first + j && group + r < n)) drop |= 1ull << j;
+  }
+  return drop;
+}
+
+// Operations a tile of a write or mixed launch takes: the launch's division,
+// unless the tree's nodes cannot hold four times its n writes. Most writes
+// then meet on a few leaves and split them one after another, and more tiles
+// only wait for each other (the first 16384 keys of an empty tree: 0.88 ms
+// with 16 to a tile, 2.3 ms with one).
+template <int NW, bool VER>
+MVBT_DEV uint32_t write_division(const tree_view<NW, VER>& tv, const work_split& ws, uint64_t n) {
+  if (ws.per_tile >= (uint32_t)NW) return NW;
+  const uint32_t per = ld_coherent((const uint64_t*)&tv.st->bump) >= 4 * n / node<NW, VER>::kData + 1 ? ws.per_tile : NW;
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)per);  // the same on every lane: kept in a scalar register
+}
+
+// Waves per SIMD the write kernels are held to: plain trees' 16-pair launch
+// needs 96 registers for five (99 cost it 5%: 500K inserts 157 -> 165 us),
+// and so does the mixed insert + range launch at 64 pairs (100 without).
+template <int NW, bool VER>
+constexpr int kWriteOccupancy = NW == 16 && !VER ? 5 : 1;
+template <int NW, bool VER, bool IR>
+constexpr int kMixedOccupancy = NW == 64 && VER && IR ? 5 : 1;
+
 template <int NW, bool VER, int OP>
-__global__ void __launch_bounds__(256) write_kernel(tree_view<NW, VER> tv, const uint32_t* keys,
-                                                    const uint32_t* values, uint64_t n) {
+__global__ void __launch_bounds__(256, (kWriteOccupancy<NW, VER>)) write_kernel(tree_view<NW, VER> tv, const uint32_t* keys,
+                                                    const uint32_t* values, uint64_t n, work_split ws) {
   tile<NW> t;
-  chunking<NW> c;
+  chunking<NW> c(write_division(tv, ws, n));
   using node_t = node<NW, VER>;
   // The top levels in LDS at 16- and 32-pair nodes: the cache saves each
   // routing group the top passes (at 16-pair nodes, one chunk per tile, it
@@ -326,16 +376,20 @@ __global__ void __launch_bounds__(256) write_kernel(tree_view<NW, VER> tv, const
   // costs a right move or two); a launch that grows a small tree routes
   // from the root.
   __shared__ route_cache<NW, 16384> rc;
-  if constexpr (NW <= 32) tv.build_route_cache(rc, 4 * n / node_t::kData + 1);
+  if constexpr (NW <= 32) tv.build_route_cache(rc, ws.cached ? 4 * n / node_t::kData + 1 : ~0ull);
   if (c.first >= n) return;
   write_ctx ctx = tv.begin_writes(t);
   ctx.exact = 1;  // ctx.want below is the chunk's exact remaining count
   for (uint64_t base = c.first; base < n; base += c.stride) {
     uint64_t i = base + t.rank();
-    bool active = i < n;
+    bool active = c.holds(base, t.rank(), n);
     uint32_t key = active ? keys[i] : 0u;
     uint32_t val = (active && OP == 0) ? values[i] : 0u;
     uint64_t q = t.ballot(active);
+    if (OP == 0 && c.per < (uint32_t)NW) {
+      q &= ~superseded<NW>(keys, base, n, c.per, t);
+      active = (q >> t.rank()) & 1;
+    }
     // Route the whole chunk first (one latency per level for all its keys),
     // then write key by key starting from the routed leaf.
     uint32_t leaf = kNone, par = kNone;
@@ -389,12 +443,12 @@ __global__ void mixed_setup_kernel(tree_state* st) {
 }
 
 template <int NW, bool VER, bool IR>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, (kMixedOccupancy<NW, VER, IR>))
     mixed_kernel(tree_view<NW, VER> tv, const uint32_t* wkeys, const uint32_t* wvals, uint64_t nw,
                  const uint32_t* rlo, const uint32_t* rhi, uint64_t nr, uint32_t* find_out, uint64_t* pairs,
-                 uint32_t* counts, uint32_t L) {
+                 uint32_t* counts, uint32_t L, work_split ws) {
   tile<NW> t;
-  chunking<NW> c;
+  chunking<NW> c(write_division(tv, ws, nw));
   const uint64_t n = nw + nr;
   // The top levels in LDS, as in write_kernel at 32-pair nodes: writes and
   // reads start below them (at every node width: on 1M-op calls it saved
@@ -403,7 +457,7 @@ __global__ void __launch_bounds__(256)
   // node (right moves follow), so the cache is used only when the tree's
   // nodes can hold four times the call's writes.
   __shared__ route_cache<NW, 16384> rc;
-  tv.build_route_cache(rc, 4 * nw / node<NW, VER>::kData + 1);
+  tv.build_route_cache(rc, ws.cached ? 4 * nw / node<NW, VER>::kData + 1 : ~0ull);
   if (c.first >= n) return;
   constexpr int OP = IR ? 0 : 1;
   const uint32_t ts = VER ? ld32_coherent(&tv.st->call_snapshot) : kLatest;
@@ -414,9 +468,10 @@ __global__ void __launch_bounds__(256)
   bool overflow = false;
   for (uint64_t base = c.first; base < n; base += c.stride) {
     const uint64_t i = base + t.rank();
-    const bool is_w = i < nw, is_r = i >= nw && i < n;
+    const bool mine = c.holds(base, t.rank(), n), is_w = mine && i < nw, is_r = mine && i >= nw;
     // writes of the chunk: routed together, leaves written together
     uint64_t q = t.ballot(is_w);
+    if (IR && q && c.per < (uint32_t)NW) q &= ~superseded<NW>(wkeys, base, nw, c.per, t);
     if (q) {
       const uint32_t key = is_w ? wkeys[i] : 0u;
       const uint32_t val = (IR && is_w) ? wvals[i] : 0u;

@@ -100,7 +100,7 @@ struct write_ctx {
                    // zero: a launch-fixed stamp (batched worker, mixed calls)
   uint32_t want;   // writes this tile still has queued (caps refills)
   uint32_t grow;   // next refill size: starts at 2, doubles up to W
-  uint32_t exact;  // nonzero: `want` is exact, version-copy refills take want + 2
+  uint32_t exact;  // nonzero: `want` is exact, version-copy refills take all of it
   uint32_t backoff;  // sleep rounds after the next failed lock (tile-uniform)
 };
 
@@ -225,7 +225,7 @@ struct tree_view : tree_ptrs {
   // stack, the rest from the never-used frontier. Returns kNone when the pool
   // is exhausted.
   // Refill size. A version copy in a write call that knows its queued writes
-  // exactly (c.exact) takes want + 2 at once: in a new epoch nearly every
+  // exactly (c.exact) takes them (and an eighth for splits) at once: in a new epoch nearly every
   // write copies its leaf, and one atomic on the shared counter then serves
   // the whole chunk. Otherwise (splits, and callers that hold one operation
   // at a time) refills grow geometrically (2, 4, 8, ... W) with demand, so a
@@ -233,7 +233,7 @@ struct tree_view : tree_ptrs {
   // slots could otherwise exhaust a nearly full pool. A plain tree writes in
   // place and allocates only to split (2 for the root). Capped at W.
   MVBT_DEV uint32_t refill_size(write_ctx& c, bool copy) const {
-    uint32_t k = VER ? c.want + 2 : 2;
+    uint32_t k = VER ? c.want + c.want / 8 : 2;
     if (!(copy && c.exact)) {
       if (k > c.grow) k = c.grow;
       if (c.grow < (uint32_t)NW) c.grow *= 2;
