@@ -1024,6 +1024,7 @@ mvbt_status mvbt_create(const mvbt_config* config, mvbt_tree** out) {
   s.root = 0;
   s.clock = 0;
   s.bump = 2;  // root + first leaf
+  s.settled = 2;
   s.capacity = cfg.pool_nodes;
   s.free_top = 0;
   s.retire_cap = cfg.retire_capacity;

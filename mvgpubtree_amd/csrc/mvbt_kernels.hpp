@@ -346,11 +346,13 @@ MVBT_DEV uint64_t superseded(const uint32_t* keys, uint64_t base, uint64_t n, ui
 // unless the tree's nodes cannot hold four times its n writes. Most writes
 // then meet on a few leaves and split them one after another, and more tiles
 // only wait for each other (the first 16384 keys of an empty tree: 0.88 ms
-// with 16 to a tile, 2.3 ms with one).
+// with 16 to a tile, 2.3 ms with one). The nodes are those of the last
+// maintenance: every wave of the launch must come to the same answer, and
+// `bump` moves while it runs.
 template <int NW, bool VER>
 MVBT_DEV uint32_t write_division(const tree_view<NW, VER>& tv, const work_split& ws, uint64_t n) {
   if (ws.per_tile >= (uint32_t)NW) return NW;
-  const uint32_t per = ld_coherent((const uint64_t*)&tv.st->bump) >= 4 * n / node<NW, VER>::kData + 1 ? ws.per_tile : NW;
+  const uint32_t per = ld_coherent((const uint64_t*)&tv.st->settled) >= 4 * n / node<NW, VER>::kData + 1 ? ws.per_tile : NW;
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)per);  // the same on every lane: kept in a scalar register
 }
 
@@ -585,6 +587,7 @@ MVBT_DEV void reclaim_prep(tree_state* st, unsigned long long end_pos, epoch_sta
   if (live > st->peak_live) st->peak_live = live;
   st->free_top = (long long)(base + count + spilled);
   st->spill_count = 0;
+  st->settled = used;
   st->scratch[0] = head;  // first ring position to copy
   st->scratch[1] = count;
   st->scratch[2] = base;

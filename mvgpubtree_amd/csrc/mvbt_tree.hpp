@@ -64,6 +64,7 @@ struct alignas(128) tree_state {
   uint32_t call_snapshot;          // snapshot reserved by the current mixed call
   uint32_t pad_call;
   unsigned long long series_count;  // reclamation epochs recorded in the memory timeline
+  unsigned long long settled;       // `bump` at the last free-list maintenance, which no write launch overlaps
 };
 
 // One entry of the memory timeline (mvbt_epoch_stat in include/mvbt.h),

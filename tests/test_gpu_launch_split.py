@@ -79,3 +79,18 @@ def test_last_of_a_repeated_key_wins_within_a_group(dev, nw, mixed):
         got = to_np(tree.find(to_dev(k, dev)))
         assert np.array_equal(got, np.array([want[x] for x in k.tolist()], np.uint32))
         assert tree.error_flags() == 0
+
+
+@pytest.mark.parametrize("n", [9_000, 10_400, 10_650, 10_900, 11_800])
+def test_insert_that_grows_the_tree_past_the_division_line(dev, n):
+    """The tree holds about 3000 nodes, a fraction of four times the call's
+    writes, and gains a third of them while the call runs: every wave must
+    divide the call the same way."""
+    rng = np.random.default_rng(n)
+    tree = mv.GpuVersionedBTree(pool_nodes=1 << 16, node_width=16)
+    keys = wl.unique_keys(rng, 30_000 + n)
+    vals = wl.value_of(keys)
+    tree.insert(to_dev(keys[:30_000], dev), to_dev(vals[:30_000], dev))
+    tree.insert(to_dev(keys[30_000:], dev), to_dev(vals[30_000:], dev))
+    assert np.array_equal(to_np(tree.find(to_dev(keys, dev))), vals)
+    assert tree.validate_tree_structure()[0] == keys.size
