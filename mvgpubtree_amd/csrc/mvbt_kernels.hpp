@@ -34,6 +34,14 @@ struct chunking {
     first = ((uint64_t)blockIdx.x * tiles_per_block + threadIdx.x / W) * per;
     stride = (uint64_t)gridDim.x * tiles_per_block * per;
   }
+  // Operations of [0, n) in the first chunks of this workgroup's tiles, tiles
+  // that hold any, and the workgroup's operations before this tile's.
+  MVBT_DEV uint32_t block_ops(uint64_t n) const {
+    const uint64_t all = (uint64_t)(blockDim.x / W) * per, b0 = blockIdx.x * all;
+    return (uint32_t)(b0 >= n ? 0 : (n - b0 < all ? n - b0 : all));
+  }
+  MVBT_DEV uint32_t block_tiles(uint64_t n) const { return (block_ops(n) + per - 1) / per; }
+  MVBT_DEV uint32_t offset() const { return threadIdx.x / W * per; }
   // Whether lane `rank` of the chunk at `base` holds operation base + rank of n.
   MVBT_DEV bool holds(uint64_t base, uint32_t rank, uint64_t n) const { return rank < per && base + rank < n; }
 };
@@ -378,10 +386,14 @@ __global__ void __launch_bounds__(256, (kWriteOccupancy<NW, VER>)) write_kernel(
   // costs a right move or two); a launch that grows a small tree routes
   // from the root.
   __shared__ route_cache<NW, 16384> rc;
+  __shared__ block_slots bs;
+  if (threadIdx.x == blockDim.x - 1) tv.reserve_block(bs, c.block_ops(n), n);
   if constexpr (NW <= 32) tv.build_route_cache(rc, ws.cached ? 4 * n / node_t::kData + 1 : ~0ull);
+  else __syncthreads();
   if (c.first >= n) return;
   write_ctx ctx = tv.begin_writes(t);
   ctx.exact = 1;  // ctx.want below is the chunk's exact remaining count
+  tv.take_reserved(ctx, bs, c.offset(), (uint32_t)(n - c.first < c.per ? n - c.first : c.per), t);
   for (uint64_t base = c.first; base < n; base += c.stride) {
     uint64_t i = base + t.rank();
     bool active = c.holds(base, t.rank(), n);
@@ -424,7 +436,7 @@ __global__ void __launch_bounds__(256, (kWriteOccupancy<NW, VER>)) write_kernel(
                             t.shfl(par, j));
     }
   }
-  tv.finish(ctx, t);
+  tv.finish_block(ctx, bs, c.block_tiles(n), t);
 }
 
 // Mixed launch (reference concurrent_insert_range_kernel btree_kernels.hpp:150-306,
@@ -459,12 +471,16 @@ __global__ void __launch_bounds__(256, (kMixedOccupancy<NW, VER, IR>))
   // node (right moves follow), so the cache is used only when the tree's
   // nodes can hold four times the call's writes.
   __shared__ route_cache<NW, 16384> rc;
+  __shared__ block_slots bs;
+  if (threadIdx.x == blockDim.x - 1) tv.reserve_block(bs, c.block_ops(nw), nw);
   tv.build_route_cache(rc, ws.cached ? 4 * nw / node<NW, VER>::kData + 1 : ~0ull);
   if (c.first >= n) return;
   constexpr int OP = IR ? 0 : 1;
   const uint32_t ts = VER ? ld32_coherent(&tv.st->call_snapshot) : kLatest;
   write_ctx ctx = tv.begin_writes(t);
   ctx.exact = 1;
+  if (c.first < nw)
+    tv.take_reserved(ctx, bs, c.offset(), (uint32_t)(nw - c.first < c.per ? nw - c.first : c.per), t);
   if (VER) ctx.cur = ts + 1;
   ctx.track = 0;  // the call's writes are stamped right after its snapshot
   bool overflow = false;
@@ -542,7 +558,7 @@ __global__ void __launch_bounds__(256, (kMixedOccupancy<NW, VER, IR>))
     }
   }
   if (t.any(overflow)) tv.flag(kErrRangeOverflow, t);
-  tv.finish(ctx, t);
+  tv.finish_block(ctx, bs, c.block_tiles(n), t);
 }
 
 // take_snapshot_kernel (btree_kernels.hpp:473-478): one lane reads the retire

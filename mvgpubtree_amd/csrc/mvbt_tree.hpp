@@ -105,6 +105,25 @@ struct write_ctx {
   uint32_t backoff;  // sleep rounds after the next failed lock (tile-uniform)
 };
 
+// Allocation and retirement of one workgroup's tiles together (in LDS). The
+// shared counters of tree_state are single addresses, whose atomics run one
+// after another at the memory side: with one to three of them per tile, a
+// launch of 16384 tiles waited about 150 us for them whatever its tiles held
+// (16K to 128K updates). The write and mixed launches therefore take the
+// version copies of all their tiles' first chunks with one reservation per
+// workgroup, and the last tile of a workgroup to finish hands over the
+// retirements and unused slots of all of them. No tile waits for another:
+// the hand-over belongs to whichever arrives last.
+struct block_slots {
+  static constexpr uint32_t kMax = 256;  // threads of a workgroup: a tile hands over at most one entry per lane
+  uint32_t ret[kMax];
+  uint32_t spare[kMax];
+  uint32_t n_ret, n_spare, arrived;
+  uint32_t got, reserved;  // slots from the free stack, and in all
+  long long top;           // free-stack top before the reservation
+  unsigned long long bump;  // first never-used index of the reservation
+};
+
 // Device pointers of one tree, independent of the node width (passed to
 // kernels by value; tree_view adds the width-specific operations).
 struct tree_ptrs {
@@ -310,6 +329,81 @@ struct tree_view : tree_ptrs {
       if (t.rank() < c.mag_n) st32_coherent(spill + s + t.rank(), c.mag);
       c.mag_n = 0;
     }
+  }
+
+  // Block-wide start of a launch's writes (one thread; the caller's next
+  // workgroup barrier publishes it): reserves `want` slots for the workgroup.
+  // Nothing is reserved unless the pool has three times the launch's `ops`
+  // writes free, so a nearly full pool is left to the tiles' own refills,
+  // which take slots only for copies they make.
+  MVBT_DEV void reserve_block(block_slots& bs, uint32_t want, uint64_t ops) const {
+    bs.n_ret = bs.n_spare = bs.arrived = 0;
+    bs.got = bs.reserved = 0;
+    if (!VER || want == 0) return;
+    const long long on_stack = (long long)ld_coherent((const uint64_t*)&st->free_top);
+    const unsigned long long used = ld_coherent((const uint64_t*)&st->bump);
+    const unsigned long long fresh = used < (unsigned long long)cap_ ? (unsigned long long)cap_ - used : 0ull;
+    if (fresh + (on_stack > 0 ? (unsigned long long)on_stack : 0ull) < 3 * ops) return;
+    const long long top = atomic_add_s64(&st->free_top, -(long long)want);
+    const uint32_t got = (uint32_t)(top < 0 ? 0 : (top > (long long)want ? (long long)want : top));
+    bs.top = top;
+    bs.got = got;
+    if (got < want) bs.bump = atomic_add64(&st->bump, (unsigned long long)(want - got));
+    bs.reserved = want;
+  }
+  // The tile's share of the reservation: entries [off, off + k), k <= W.
+  MVBT_DEV void take_reserved(write_ctx& c, const block_slots& bs, uint32_t off, uint32_t k, const tile_t& t) const {
+    const uint32_t r = t.rank(), e = off + r;
+    uint32_t idx = kNone;
+    if (bs.reserved && r < k) {
+      if (e < bs.got) {
+        idx = ld32_coherent(free_stack + (bs.top - 1 - (long long)e));
+      } else {
+        const unsigned long long f = bs.bump + (e - bs.got);
+        idx = f < (unsigned long long)cap_ ? (uint32_t)f : kNone;
+      }
+    }
+    c.mag = idx;  // valid lanes are a prefix, as in refill()
+    c.mag_n = (uint32_t)__builtin_popcountll(t.ballot(idx != kNone));
+  }
+  // finish() through the workgroup: the last of its `tiles` tiles to arrive
+  // enters every retirement in the ring and every unused slot in the spill
+  // list. Each tile calls it once, after its last write.
+  MVBT_DEV void finish_block(write_ctx& c, block_slots& bs, uint32_t tiles, const tile_t& t) const {
+    const uint32_t r = t.rank();
+    uint32_t ro = 0, so = 0;
+    if (t.leader()) {
+      if (c.ret_n) ro = __hip_atomic_fetch_add(&bs.n_ret, c.ret_n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (c.mag_n) so = __hip_atomic_fetch_add(&bs.n_spare, c.mag_n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    ro = t.shfl(ro, 0);
+    so = t.shfl(so, 0);
+    if (r < c.ret_n) bs.ret[ro + r] = c.ret;
+    if (r < c.mag_n) bs.spare[so + r] = c.mag;
+    uint32_t before = 0;
+    if (t.leader()) before = __hip_atomic_fetch_add(&bs.arrived, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (t.shfl(before, 0) + 1 != tiles) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    const uint32_t nr = bs.n_ret, ns = bs.n_spare;
+    unsigned long long pos = 0, head = 0, s = 0;
+    if (t.leader()) {
+      if (nr) {
+        pos = atomic_add64(&st->retire_tail, (unsigned long long)nr);
+        head = __hip_atomic_load(&st->retire_head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      if (ns) s = atomic_add64(&st->spill_count, (unsigned long long)ns);
+    }
+    pos = t.shfl64(pos, 0);
+    head = t.shfl64(head, 0);
+    s = t.shfl64(s, 0);
+    bool over = false;
+    for (uint32_t i = r; i < nr; i += NW) {
+      const unsigned long long p = pos + i;
+      if (p - head < retire_cap) st32_coherent(retire_ring + (p & (retire_cap - 1)), bs.ret[i]);
+      else over = true;  // as in flush_retired()
+    }
+    for (uint32_t i = r; i < ns; i += NW) st32_coherent(spill + s + i, bs.spare[i]);
+    if (t.any(over)) flag(kErrRetireOverflow, t);
   }
 
   // ---- locks (reference versioned_node.hpp:528-568; here try-lock only) ----

@@ -94,3 +94,32 @@ def test_insert_that_grows_the_tree_past_the_division_line(dev, n):
     tree.insert(to_dev(keys[30_000:], dev), to_dev(vals[30_000:], dev))
     assert np.array_equal(to_np(tree.find(to_dev(keys, dev))), vals)
     assert tree.validate_tree_structure()[0] == keys.size
+
+@pytest.mark.parametrize("nw", [16, 32, 64])
+@pytest.mark.parametrize("spare", [200, 30_000])
+def test_slots_of_a_workgroup_are_all_accounted_for(dev, nw, spare):
+    """Updates that copy every leaf, no leaf twice, and absent keys that copy
+    none: after reclamation the pool holds the tree's nodes and nothing else,
+    both where the pool allows the workgroups' reservations (spare well above
+    three slots a write) and where it does not."""
+    rng = np.random.default_rng(nw + spare)
+    keys = wl.unique_keys(rng, 60_000)
+    probe = mv.GpuVersionedBTree(pool_nodes=1 << 16, node_width=nw)
+    probe.bulk_build(to_dev(np.sort(keys), dev), to_dev(wl.value_of(np.sort(keys)), dev))
+    nodes = probe.memory_stats().live_nodes
+    tree = mv.GpuVersionedBTree(pool_nodes=nodes + spare, node_width=nw)
+    ks = np.sort(keys)
+    tree.bulk_build(to_dev(ks, dev), to_dev(wl.value_of(ks), dev))
+    absent = wl.absent_keys(rng, 3000, ks)
+    for r in range(6):
+        s = tree.take_snapshot()
+        some = rng.choice(ks, size=150, replace=False)
+        tree.insert(to_dev(some, dev), to_dev(np.full(150, r + 1, np.uint32), dev))
+        tree.erase(to_dev(absent, dev))  # copies nothing
+        tree.release_snapshot(s)
+        tree.reclaim()
+        assert np.all(to_np(tree.find(to_dev(some, dev))) == r + 1)
+        assert tree.error_flags() == 0
+        m = tree.memory_stats()
+        assert m.live_nodes == nodes and m.retired_pending == 0
+    assert tree.validate_tree_structure()[0] == ks.size
