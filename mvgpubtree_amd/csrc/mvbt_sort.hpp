@@ -31,6 +31,10 @@ MVBT_DEV void segment_of(uint32_t n, uint32_t g, uint32_t G, uint32_t& a, uint32
   b = (uint64_t)a + seg < n ? a + seg : n;
 }
 
+__global__ void set_word_kernel(uint32_t* p, uint32_t v) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *p = v;
+}
+
 __global__ void __launch_bounds__(kSortBlock)
     radix_hist_kernel(const uint32_t* keys, const uint32_t* n_ptr, uint32_t shift, uint32_t* hist) {
   __shared__ uint32_t h[kRadix];
