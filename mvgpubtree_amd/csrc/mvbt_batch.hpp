@@ -264,6 +264,61 @@ __global__ void batch_count_kernel(batch_job* job, tree_state* st) {
   }
 }
 
+// 2 (sorted form). Each operation's batch, the call's write count and the
+// checks, over equal slices of the operations: the batches differ in size by
+// three orders of magnitude, and a workgroup to a batch waits for the largest
+// (480 batches of 4M operations: 129 us). A slice's batches are looked up in
+// a copy of their offsets in LDS where it has at most kSliceBatches of them.
+constexpr uint32_t kSliceBatches = 2048;
+MVBT_DEV uint32_t batch_in(const unsigned long long* offsets, uint32_t lo, uint32_t hi, unsigned long long i) {
+  while (hi - lo > 1) {  // offsets[lo] <= i < offsets[hi]
+    const uint32_t mid = (lo + hi) >> 1;
+    if (offsets[mid] <= i) lo = mid;
+    else hi = mid;
+  }
+  return lo;
+}
+__global__ void __launch_bounds__(256) batch_slice_kernel(batch_job* job, tree_state* st) {
+  __shared__ unsigned long long off[kSliceBatches + 1];
+  __shared__ uint32_t bounds[2], part[4];
+  if (ld32_coherent(&job->bad)) return;  // offsets disagree with the op count
+  const uint32_t nb = job->nb, tid = threadIdx.x;
+  const unsigned long long first = job->first_op, n = job->nops - first;
+  bool bad = false;
+  for (uint32_t b = blockIdx.x * 256 + tid; b < nb; b += gridDim.x * 256) bad |= job->offsets[b + 1] < job->offsets[b];
+  const unsigned long long per = (n + gridDim.x - 1) / gridDim.x, a = first + per * blockIdx.x;
+  const unsigned long long e = a + per < first + n ? a + per : first + n;
+  uint32_t c = 0;
+  if (a < e) {
+    if (tid < 2) bounds[tid] = batch_in(job->offsets, 0, nb, tid ? e - 1 : a);
+    __syncthreads();
+    // (offsets out of order may give any batches here: the call is rejected)
+    const uint32_t b0 = bounds[0], b1 = bounds[1] < b0 ? b0 : bounds[1];
+    const bool local = b1 - b0 < kSliceBatches;
+    if (local) {
+      for (uint32_t k = tid; k <= b1 - b0 + 1; k += 256) off[k] = job->offsets[b0 + k];
+      __syncthreads();
+    }
+    for (unsigned long long i = a + tid; i < e; i += 256) {
+      const uint32_t ty = job->ops[i].type;
+      c += ty == kOpInsert || ty == kOpErase ? 1u : 0u;
+      bad |= ty > kOpRange;
+      job->op_batch[i - first] = local ? b0 + batch_in(off, 0, b1 - b0 + 1, i) : batch_in(job->offsets, b0, b1 + 1, i);
+    }
+  }
+  if (bad) {
+    atomic_or32(&job->bad, 1u);
+    atomic_or32(&st->error_flags, kErrBadBatch);
+  }
+  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+  if ((tid & 63) == 0) part[tid >> 6] = c;
+  __syncthreads();
+  if (tid == 0) {
+    const uint32_t tot = part[0] + part[1] + part[2] + part[3];
+    if (tot) atomic_add32(&job->total_writes, tot);
+  }
+}
+
 // 2'. The conflict table's size: the smallest power of two >= twice the
 // call's writes (at least 1024, at most its capacity), so a table that fits
 // the caches serves a call whose operations are mostly reads.
@@ -800,6 +855,14 @@ __global__ void __launch_bounds__(kSortBlock) batch_split_kernel(batch_job* job)
   }
 }
 
+// How the sorted form's kernels divide n operations, a count only the device
+// knows: one to a tile while that leaves tiles idle, then as few as keep
+// `tiles` of them busy (as split_for does for the plain launches).
+MVBT_DEV uint32_t per_tile(uint32_t n, uint32_t tiles, uint32_t width) {
+  const uint32_t p = (n + tiles - 1) / tiles;
+  return p < 1 ? 1u : p < width ? p : width;
+}
+
 // 7. Routes every write to its leaf: sort key = leaf (cap_ for a key that is
 // not routed: reserved keys, which fail in the write pass), payload = the
 // write's position in w_rel; the parent goes to w_par. T: routing tile
@@ -809,10 +872,11 @@ __global__ void __launch_bounds__(256) batch_route_kernel(tree_ptrs tp, batch_jo
   if (ld32_coherent(&job->bad)) return;
   const tree_view<NW, true> tv(tp);
   tile<T> t;
-  chunking<T> c;
-  __shared__ route_cache<NW, kRangeCacheBytes> rc;
-  tv.build_route_cache(rc);
   const uint32_t n = job->n_writes;
+  chunking<T> c(per_tile(n, gridDim.x * (blockDim.x / T) / 2, T));  // half the grid's tiles are resident
+  if (c.block_ops(n) == 0) return;
+  __shared__ route_cache<NW, kRangeCacheBytes> rc;
+  tv.build_route_cache(rc, c.per >= kCachedFrom ? 0ull : ~0ull);
   const op_record* ops = job->ops + job->first_op;
   const uint32_t* w_rel = job->w_rel;
   uint32_t* hint = job->sort_k[0];
@@ -820,7 +884,7 @@ __global__ void __launch_bounds__(256) batch_route_kernel(tree_ptrs tp, batch_jo
   uint32_t* w_par = job->w_par;
   for (uint64_t base = c.first; base < n; base += c.stride) {
     const uint64_t i = base + t.rank();
-    const bool act = i < n;
+    const bool act = c.holds(base, t.rank(), n);
     const uint32_t key = act ? ops[w_rel[i]].key : 0u;
     const bool go = act && valid_key(key);
     const uint64_t q = t.ballot(go);
@@ -978,9 +1042,9 @@ __global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, b
   if (ld32_coherent(&job->bad)) return;
   const tree_view<NW, true> tv(tp);
   tile<NW> t;
-  chunking<NW> c;
   const uint32_t r = t.rank();
   const uint32_t n = job->n_writes;
+  const chunking<NW> c(per_tile(n, gridDim.x * (blockDim.x / NW), NW));
   const uint32_t* hint = job->sort_k[which];
   const uint32_t* const* g = job->gat;  // the writes' fields in sorted order
   uint32_t* results = job->results + job->first_op;
@@ -990,12 +1054,12 @@ __global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, b
   ctx.track = 0;  // stamps are fixed per batch: clock0 + b + 1
   for (uint64_t p = c.first; p < n; p += c.stride) {
     uint64_t i = p + r;
-    bool start = i < n && (i == 0 || hint[i] != hint[i - 1]);
+    bool start = c.holds(p, r, n) && (i == 0 || hint[i] != hint[i - 1]);
     const uint64_t starts = t.ballot(start);
     if (!starts) continue;  // the window lies inside a group that started earlier
-    // sub-windows of NW positions from the first group start in the window to
+    // sub-windows of NW positions from the first group start in the window (of c.per positions) to
     // the first group start at or past its end
-    const uint64_t wend = p + NW;
+    const uint64_t wend = p + c.per;
     for (uint64_t a = p + (uint64_t)lowest_bit(starts);; a += NW) {
       i = a + r;
       const bool in = i < n;
@@ -1071,10 +1135,11 @@ batch_sorted_find_kernel(tree_ptrs tp, const batch_job* job) {
   if (ld32_coherent(&job->bad)) return;
   const tree_view<NW, true> tv(tp);
   tile<T> t;
-  chunking<T> c;
-  __shared__ route_cache<NW, kFindCacheBytes> rc;
-  tv.build_route_cache(rc);
   const uint32_t n = job->n_finds;
+  chunking<T> c(per_tile(n, gridDim.x * (blockDim.x / T), T));
+  if (c.block_ops(n) == 0) return;
+  __shared__ route_cache<NW, kFindCacheBytes> rc;
+  tv.build_route_cache(rc, c.per >= kCachedFrom ? 0ull : ~0ull);
   const uint32_t* list = job->rd_find;
   const uint32_t* op_batch = job->op_batch;
   const op_record* ops = job->ops + job->first_op;
@@ -1082,7 +1147,7 @@ batch_sorted_find_kernel(tree_ptrs tp, const batch_job* job) {
   const uint32_t clock0 = job->clock0;
   for (uint64_t base = c.first; base < n; base += c.stride) {
     const uint64_t i = base + t.rank();
-    const bool act = i < n;
+    const bool act = c.holds(base, t.rank(), n);
     const uint32_t rel = act ? list[i] : 0u;
     const uint32_t key = act ? ops[rel].key : 0u;
     const uint32_t ts = act ? clock0 + op_batch[rel] : 0u;
@@ -1116,10 +1181,11 @@ __global__ void __launch_bounds__(256) batch_sorted_range_kernel(tree_ptrs tp, c
   using rc_t = route_cache<NW, kRangeCacheBytes>;
   const tree_view<NW, true> tv(tp);
   tile<T> t;
-  chunking<T> c;
-  __shared__ rc_t rc;
-  tv.build_route_cache(rc);
   const uint32_t n = job->n_ranges, L = job->L;
+  chunking<T> c(per_tile(n, gridDim.x * (blockDim.x / T) / 2, T));  // half the grid's tiles are resident
+  if (c.block_ops(n) == 0) return;
+  __shared__ rc_t rc;
+  tv.build_route_cache(rc, c.per >= kCachedFrom ? 0ull : ~0ull);
   const uint32_t* list = job->rd_range;
   const uint32_t* op_batch = job->op_batch;
   const op_record* ops = job->ops + job->first_op;
@@ -1130,7 +1196,7 @@ __global__ void __launch_bounds__(256) batch_sorted_range_kernel(tree_ptrs tp, c
   bool overflow = false, bad_slot = false;
   for (uint64_t base = c.first; base < n; base += c.stride) {
     const uint64_t i = base + t.rank();
-    const bool act = i < n;
+    const bool act = c.holds(base, t.rank(), n);
     const uint32_t rel = act ? list[i] : 0u;
     op_record op{};
     if (act) op = ops[rel];

@@ -176,11 +176,6 @@ uint32_t grid_for(const mvbt_tree* t, uint64_t n, uint32_t width, uint32_t per, 
 // with fewer to a tile a small launch waits for fewer chains: on MI355X (32
 // pairs per node) 64 finds took 39.2 us with 16 to a tile and 8.5 with one,
 // 1000 updates 82 and 21, 64K range queries 65 and 29 (4 to a tile).
-// The top levels are copied to LDS only where a tile then routes at least
-// kCachedFrom operations through them: the copy takes 5-7 us, and the walk it
-// shortens is read once. 128K finds (4 to a tile) 26.3 us without it and 30.1
-// with, 256K (8) 45.2 and 41.6.
-constexpr uint32_t kCachedFrom = 5;
 work_split split_for(const mvbt_tree* t, uint64_t n, uint32_t width, int waves) {
   const uint64_t tiles = (uint64_t)t->num_cus * (uint64_t)waves * (64 / width);
   work_split ws;
@@ -953,7 +948,9 @@ mvbt_status build_graph(mvbt_tree* t, const batch_params& bp) {
   void* count_args[] = {&job, &st};
   MVBT_HIP(add(reinterpret_cast<void*>(&batch_setup_kernel), 1, 64, setup_args));
   t->graph_setup[gi] = node;
-  MVBT_HIP(add(reinterpret_cast<void*>(&batch_count_kernel), t->num_cus * 4, kBlock, count_args));
+  MVBT_HIP(add(t->eff_mode == 2 ? reinterpret_cast<void*>(&batch_slice_kernel)
+                                : reinterpret_cast<void*>(&batch_count_kernel),
+               t->num_cus * 4, kBlock, count_args));
   MVBT_HIP(add(reinterpret_cast<void*>(&batch_mask_kernel), 1, 64, job_args));
   MVBT_HIP(add(reinterpret_cast<void*>(&batch_clear_kernel), t->num_cus * 4, kBlock, job_args));
   MVBT_HIP(add(reinterpret_cast<void*>(&batch_conflict_kernel), t->num_cus * 8, kBlock, count_args));
@@ -1521,7 +1518,10 @@ mvbt_status mvbt_run_batches(mvbt_tree* t, const mvbt_op* ops, uint64_t num_ops,
     MVBT_HIP(hipGraphLaunch(t->graph_exec[gi], s));
   } else {
     hipLaunchKernelGGL(batch_setup_kernel, dim3(1), dim3(64), 0, s, t->job, t->st, p);
-    hipLaunchKernelGGL(batch_count_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job, t->st);
+    if (t->eff_mode == 2)
+      hipLaunchKernelGGL(batch_slice_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job, t->st);
+    else
+      hipLaunchKernelGGL(batch_count_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job, t->st);
     hipLaunchKernelGGL(batch_mask_kernel, dim3(1), dim3(64), 0, s, t->job);
     hipLaunchKernelGGL(batch_clear_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job);
     hipLaunchKernelGGL(batch_conflict_kernel, dim3(t->num_cus * 8), dim3(kBlock), 0, s, t->job, t->st);
@@ -1626,7 +1626,7 @@ mvbt_status mvbt_run_batches_noalloc(mvbt_tree* t, const mvbt_op* ops, uint64_t 
   p.reclaim = may_reclaim_in_call(t, 0) ? 1u : 0u;
   hipLaunchKernelGGL(batch_bind_kernel, dim3(1), dim3(64), 0, s, job, l);
   hipLaunchKernelGGL(batch_setup_kernel, dim3(1), dim3(64), 0, s, job, t->st, p);
-  hipLaunchKernelGGL(batch_count_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, job, t->st);
+  hipLaunchKernelGGL(batch_slice_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, job, t->st);
   hipLaunchKernelGGL(batch_mask_kernel, dim3(1), dim3(64), 0, s, job);
   hipLaunchKernelGGL(batch_clear_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, job);
   hipLaunchKernelGGL(batch_conflict_kernel, dim3(t->num_cus * 8), dim3(kBlock), 0, s, job, t->st);
