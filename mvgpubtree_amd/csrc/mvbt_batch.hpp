@@ -42,6 +42,14 @@ struct op_record {
   uint32_t type, key, arg, slot;
 };
 
+// A write of the sorted form: one 16-byte record, so that the gather into
+// sorted order touches one line per write.
+struct alignas(16) write_rec {
+  uint32_t key, arg;
+  uint32_t rel;    // index - first_op, bit 31: erase
+  uint32_t batch;
+};
+
 struct alignas(128) batch_job {
   // per-call parameters (written by batch_setup_kernel)
   const op_record* ops;
@@ -73,19 +81,18 @@ struct alignas(128) batch_job {
   int32_t frontier[8 * 32];
   // Sorted form (worker mode 2): library-owned scratch, one entry per
   // operation unless stated.
-  uint32_t* w_rel;       // write operations (index - first_op), in operation order
-  uint32_t* w_par;       // parent hint of each write (indexed like w_rel)
-  uint32_t* sort_k[2];   // leaf hints (sort keys), two buffers
-  uint32_t* sort_v[2];   // positions in w_rel (sort payloads), two buffers
-  uint32_t* rd_find;     // find operations (index - first_op), any order
-  uint32_t* rd_range;    // range operations (index - first_op), any order
-  uint32_t* seg;         // per class (writes, finds, ranges) kSortSegments segment counts
+  uint32_t* list;        // the call's finds, then its ranges (index - first_op), in operation order
+  write_rec* writes;     // the call's writes, in operation order
+  uint32_t* w_par;       // parent hint of each write of the window
+  uint32_t* sort_k[2];   // leaf hints (sort keys), two buffers; the spare one then holds the
+                         // sorted writes' parent hints
+  uint32_t* sort_v[2];   // positions in the window's writes (sort payloads), two buffers; the
+                         // spare one then holds the sorted writes' copy slots
+  write_rec* sorted;     // the window's writes in sorted order
+  uint32_t* seg;         // segment counts: kOpClasses * kSliceWaves
   uint32_t* hist;        // kRadix * kSortSegments histogram + kRadix digit totals
-  // the sorted writes' fields in sorted order (batch_gather_kernel): key,
-  // value, index - first_op (bit 31: erase), batch, parent hint, copy slot
-  uint32_t* gat[6];
   // counts of the current call (zeroed by batch_setup_kernel), one line
-  uint32_t n_writes;
+  uint32_t n_writes;     // of the current window
   uint32_t n_finds;
   uint32_t n_ranges;
   uint32_t n_epochs;     // (leaf, batch) groups of the sorted writes: one planned copy slot each
@@ -97,13 +104,12 @@ struct alignas(128) batch_job {
   unsigned long long cp_bump;       // first never-used index of the reservation
   unsigned long long cp_ring;       // first retire-ring position of the reservation
   // windows of the sorted form: the call's batches in `windows` consecutive
-  // groups of about equal operation count; [w_lo, w_hi) = the current
-  // window's operations (index - first_op)
+  // groups of about equal operation count
   uint32_t windows;
   uint32_t reclaim;
-  uint32_t w_lo;
-  uint32_t w_hi;
-  unsigned long long pad4[7];
+  uint32_t first[3];     // the window's first write, find and range in their part of `list`
+  uint32_t total[3];     // the call's writes, finds and ranges
+  unsigned long long pad4[5];
 };
 constexpr uint32_t kFrontierCopies = 8;
 
@@ -151,8 +157,7 @@ __global__ void batch_setup_kernel(batch_job* job, tree_state* st, batch_params 
   job->n_ranges = 0;
   job->windows = p.windows > 0 ? p.windows : 1u;
   job->reclaim = p.reclaim;
-  job->w_lo = 0;
-  job->w_hi = ok ? (uint32_t)(last - first) : 0u;
+  if (p.base_out) *p.base_out = job->clock0;  // clock0 goes back to the caller
   if (!ok) atomic_or32(&st->error_flags, kErrBadBatch);
   for (uint32_t c = 0; c < kFrontierCopies; ++c) job->frontier[c * 32] = -1;
 }
@@ -160,13 +165,14 @@ __global__ void batch_setup_kernel(batch_job* job, tree_state* st, batch_params 
 // 0. Points a job descriptor at its scratch arrays from the device side (the
 // allocation-free entry point: the job and its scratch all lie in one static
 // device array, so no host copy is needed).
+constexpr uint32_t kSortedPtrs = 10;  // list .. hist of batch_job
 struct scratch_layout {
   uint32_t* nwrites;
   uint32_t* done;
   int32_t* advance;
   uint32_t* hash;
   uint32_t* op_batch;
-  uint32_t* sorted[16];  // w_rel, w_par, sort_k[0..1], sort_v[0..1], rd_find, rd_range, seg, hist, gat[0..5]
+  uint32_t* sorted[kSortedPtrs];  // list .. hist, in the order of batch_job
 };
 __global__ void batch_bind_kernel(batch_job* job, scratch_layout l) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
@@ -175,17 +181,16 @@ __global__ void batch_bind_kernel(batch_job* job, scratch_layout l) {
   job->advance = l.advance;
   job->hash = l.hash;
   job->op_batch = l.op_batch;
-  job->w_rel = l.sorted[0];
-  job->w_par = l.sorted[1];
-  job->sort_k[0] = l.sorted[2];
-  job->sort_k[1] = l.sorted[3];
-  job->sort_v[0] = l.sorted[4];
-  job->sort_v[1] = l.sorted[5];
-  job->rd_find = l.sorted[6];
-  job->rd_range = l.sorted[7];
+  job->list = l.sorted[0];
+  job->writes = reinterpret_cast<write_rec*>(l.sorted[1]);
+  job->w_par = l.sorted[2];
+  job->sort_k[0] = l.sorted[3];
+  job->sort_k[1] = l.sorted[4];
+  job->sort_v[0] = l.sorted[5];
+  job->sort_v[1] = l.sorted[6];
+  job->sorted = reinterpret_cast<write_rec*>(l.sorted[7]);
   job->seg = l.sorted[8];
   job->hist = l.sorted[9];
-  for (int k = 0; k < 6; ++k) job->gat[k] = l.sorted[10 + k];
 }
 
 // 1'. Clears the conflict table (a fill kernel, so the launch graph holds no
@@ -264,12 +269,20 @@ __global__ void batch_count_kernel(batch_job* job, tree_state* st) {
   }
 }
 
-// 2 (sorted form). Each operation's batch, the call's write count and the
-// checks, over equal slices of the operations: the batches differ in size by
-// three orders of magnitude, and a workgroup to a batch waits for the largest
-// (480 batches of 4M operations: 129 us). A slice's batches are looked up in
-// a copy of their offsets in LDS where it has at most kSliceBatches of them.
+// Operation classes of the sorted form: writes (insert, erase), finds, ranges.
+MVBT_DEV uint32_t op_class(uint32_t ty) {
+  return (ty == kOpInsert || ty == kOpErase) ? 0u : ty == kOpFind ? 1u : ty == kOpRange ? 2u : 3u;
+}
+constexpr uint32_t kOpClasses = 3;
+
+// 2 (sorted form). Each operation's batch, the checks, and the operations of
+// each class, over equal slices of the operations, one to a wave
+// (seg[class * kSliceWaves + slice]): the batches differ in size by three
+// orders of magnitude, and a workgroup to a batch waits for the largest (480
+// batches of 4M operations: 129 us). A workgroup looks its slices' batches up
+// in a copy of their offsets in LDS where it has at most kSliceBatches.
 constexpr uint32_t kSliceBatches = 2048;
+constexpr uint32_t kSliceBlocks = 1024, kSliceWaves = kSliceBlocks * (kSortBlock / 64);
 MVBT_DEV uint32_t batch_in(const unsigned long long* offsets, uint32_t lo, uint32_t hi, unsigned long long i) {
   while (hi - lo > 1) {  // offsets[lo] <= i < offsets[hi]
     const uint32_t mid = (lo + hi) >> 1;
@@ -278,48 +291,142 @@ MVBT_DEV uint32_t batch_in(const unsigned long long* offsets, uint32_t lo, uint3
   }
   return lo;
 }
-__global__ void __launch_bounds__(256) batch_slice_kernel(batch_job* job, tree_state* st) {
+__global__ void __launch_bounds__(kSortBlock) batch_slice_kernel(batch_job* job, tree_state* st) {
+  constexpr uint32_t kWaves = kSortBlock / 64;
   __shared__ unsigned long long off[kSliceBatches + 1];
-  __shared__ uint32_t bounds[2], part[4];
-  if (ld32_coherent(&job->bad)) return;  // offsets disagree with the op count
-  const uint32_t nb = job->nb, tid = threadIdx.x;
-  const unsigned long long first = job->first_op, n = job->nops - first;
+  __shared__ uint32_t bounds[2];
+  const uint32_t nb = job->nb, tid = threadIdx.x, lane = tid & 63, w = blockIdx.x * kWaves + tid / 64;
+  const unsigned long long first = job->first_op;
+  const uint32_t n = (uint32_t)(job->nops - first);  // 0 if the offsets disagree with the op count
   bool bad = false;
-  for (uint32_t b = blockIdx.x * 256 + tid; b < nb; b += gridDim.x * 256) bad |= job->offsets[b + 1] < job->offsets[b];
-  const unsigned long long per = (n + gridDim.x - 1) / gridDim.x, a = first + per * blockIdx.x;
-  const unsigned long long e = a + per < first + n ? a + per : first + n;
-  uint32_t c = 0;
+  if (n)
+    for (uint32_t b = blockIdx.x * kSortBlock + tid; b < nb; b += gridDim.x * kSortBlock)
+      bad |= job->offsets[b + 1] < job->offsets[b];
+  uint32_t a, e, unused, c[kOpClasses] = {0, 0, 0};
+  segment_of(n, blockIdx.x * kWaves, kSliceWaves, a, unused);
+  segment_of(n, blockIdx.x * kWaves + kWaves - 1, kSliceWaves, unused, e);
   if (a < e) {
-    if (tid < 2) bounds[tid] = batch_in(job->offsets, 0, nb, tid ? e - 1 : a);
+    if (tid < 2) bounds[tid] = batch_in(job->offsets, 0, nb, first + (tid ? e - 1 : a));
     __syncthreads();
     // (offsets out of order may give any batches here: the call is rejected)
     const uint32_t b0 = bounds[0], b1 = bounds[1] < b0 ? b0 : bounds[1];
     const bool local = b1 - b0 < kSliceBatches;
     if (local) {
-      for (uint32_t k = tid; k <= b1 - b0 + 1; k += 256) off[k] = job->offsets[b0 + k];
+      for (uint32_t k = tid; k <= b1 - b0 + 1; k += kSortBlock) off[k] = job->offsets[b0 + k];
       __syncthreads();
     }
-    for (unsigned long long i = a + tid; i < e; i += 256) {
-      const uint32_t ty = job->ops[i].type;
-      c += ty == kOpInsert || ty == kOpErase ? 1u : 0u;
-      bad |= ty > kOpRange;
-      job->op_batch[i - first] = local ? b0 + batch_in(off, 0, b1 - b0 + 1, i) : batch_in(job->offsets, b0, b1 + 1, i);
+    segment_of(n, w, kSliceWaves, a, e);
+    for (uint32_t i0 = a; i0 < e; i0 += 64) {
+      const uint32_t i = i0 + lane;
+      uint32_t k = kOpClasses;
+      if (i < e) {
+        k = op_class(job->ops[first + i].type);
+        bad |= k == kOpClasses;
+        job->op_batch[i] =
+            local ? b0 + batch_in(off, 0, b1 - b0 + 1, first + i) : batch_in(job->offsets, b0, b1 + 1, first + i);
+      }
+#pragma unroll
+      for (uint32_t q = 0; q < kOpClasses; ++q) c[q] += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(k == q));
+    }
+  }
+  if (lane < kOpClasses) job->seg[lane * kSliceWaves + w] = lane == 0 ? c[0] : lane == 1 ? c[1] : c[2];
+  if (bad) {
+    atomic_or32(&job->bad, 1u);
+    atomic_or32(&st->error_flags, kErrBadBatch);
+  }
+}
+
+// 2b. One workgroup per class: slice counts to positions, the call's totals,
+// and (a call in one window) the window's counts. The first one also sizes
+// the conflict table: the smallest power of two >= twice the call's writes
+// (at least 1024, at most its capacity), so a table that fits the caches
+// serves a call whose operations are mostly reads.
+__global__ void __launch_bounds__(kSortBlock) batch_class_scan_kernel(batch_job* job) {
+  static_assert(kSliceWaves <= kScanMax, "one row");
+  __shared__ scan_lds l;
+  const uint32_t q = blockIdx.x;
+  const uint32_t total = scan_row(job->seg + q * kSliceWaves, kSliceWaves, l);
+  if (threadIdx.x != kSortBlock - 1) return;
+  job->total[q] = total;
+  job->first[q] = 0;
+  (q == 0 ? job->n_writes : q == 1 ? job->n_finds : job->n_ranges) = total;
+  if (q == 0) {
+    unsigned long long e = 1024;
+    while (e < 2ull * total) e *= 2;
+    const unsigned long long cap = (unsigned long long)job->hash_cap_mask + 1;
+    job->hash_mask = (uint32_t)((e < cap ? e : cap) - 1);
+  }
+}
+
+// 2c. Every class to its list, in operation order (a stable scatter per slice;
+// no shared counter); the conflict table is cleared.
+__global__ void __launch_bounds__(kSortBlock) batch_split_kernel(batch_job* job) {
+  if (ld32_coherent(&job->bad)) return;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, w = blockIdx.x * (kSortBlock / 64) + tid / 64;
+  const uint32_t n = (uint32_t)(job->nops - job->first_op);
+  const op_record* ops = job->ops + job->first_op;
+  const uint32_t* op_batch = job->op_batch;
+  const uint64_t below = (1ull << lane) - 1;
+  uint32_t a, e, run[kOpClasses];
+  segment_of(n, w, kSliceWaves, a, e);
+#pragma unroll
+  for (uint32_t q = 0; q < kOpClasses; ++q)
+    run[q] = job->seg[q * kSliceWaves + w] + (q == 2 ? job->total[1] : 0u);  // ranges behind the finds
+  for (uint32_t i0 = a; i0 < e; i0 += 64) {
+    const uint32_t i = i0 + lane;
+    op_record o{};
+    uint32_t k = kOpClasses, b = 0;
+    if (i < e) {
+      o = ops[i];
+      b = op_batch[i];
+      k = op_class(o.type);
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < kOpClasses; ++q) {
+      const uint64_t m = __builtin_amdgcn_ballot_w64(k == q);
+      const uint32_t pos = run[q] + (uint32_t)__builtin_popcountll(m & below);
+      if (k == q) {
+        if (q == 0) job->writes[pos] = write_rec{o.key, o.arg, i | (o.type == kOpErase ? 0x80000000u : 0u), b};
+        else job->list[pos] = i;
+      }
+      run[q] += (uint32_t)__builtin_popcountll(m);
+    }
+  }
+  const uint32_t mask = job->hash_mask;
+  for (uint32_t i = blockIdx.x * kSortBlock + tid; i <= mask; i += gridDim.x * kSortBlock) job->hash[i] = 0;
+}
+
+// 2d. Distinct write keys per batch: every write of a valid key claims
+// (batch, key) in the conflict table (an entry is 1 + the write's position);
+// a second claim rejects the call. The table has at least twice as many
+// entries as the call has writes, so a free entry always exists.
+__global__ void __launch_bounds__(kSortBlock) batch_claim_kernel(batch_job* job, tree_state* st) {
+  if (ld32_coherent(&job->bad)) return;
+  const uint32_t n = job->total[0], mask = job->hash_mask;
+  const write_rec* writes = job->writes;
+  uint32_t* table = job->hash;
+  bool bad = false;
+  for (uint32_t i = blockIdx.x * kSortBlock + threadIdx.x; i < n; i += gridDim.x * kSortBlock) {
+    const uint32_t key = writes[i].key, b = writes[i].batch;
+    if (!valid_key(key)) continue;
+    uint32_t h = conflict_hash(key, b) & mask;
+    for (uint32_t probe = 0; probe <= mask; ++probe) {
+      const uint32_t cur = atomic_cas32(table + h, 0u, i + 1);  // most entries are free: no look before
+      if (cur == 0) break;
+      if (writes[cur - 1].key == key && writes[cur - 1].batch == b) {
+        bad = true;
+        break;
+      }
+      h = (h + 1) & mask;
     }
   }
   if (bad) {
     atomic_or32(&job->bad, 1u);
     atomic_or32(&st->error_flags, kErrBadBatch);
   }
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-  if ((tid & 63) == 0) part[tid >> 6] = c;
-  __syncthreads();
-  if (tid == 0) {
-    const uint32_t tot = part[0] + part[1] + part[2] + part[3];
-    if (tot) atomic_add32(&job->total_writes, tot);
-  }
 }
 
-// 2'. The conflict table's size: the smallest power of two >= twice the
+// 2' (modes 0 and 1). The conflict table's size: the smallest power of two >= twice the
 // call's writes (at least 1024, at most its capacity), so a table that fits
 // the caches serves a call whose operations are mostly reads.
 __global__ void batch_mask_kernel(batch_job* job) {
@@ -364,11 +471,6 @@ __global__ void batch_frontier_kernel(batch_job* job) {
     while (j < nb && job->nwrites[j] == 0) ++j;
     for (uint32_t c = 0; c < kFrontierCopies; ++c) job->frontier[c * 32] = (int32_t)j - 1;
   }
-}
-
-// 5. Hands clock0 back.
-__global__ void batch_finish_kernel(batch_job* job) {
-  if (threadIdx.x == 0 && blockIdx.x == 0 && job->base_out) *job->base_out = job->clock0;
 }
 
 // Batch of op i (offsets[0] <= i < offsets[nb]), by bisection.
@@ -748,16 +850,24 @@ MVBT_DEV uint32_t window_start(const batch_job* job, uint32_t k) {
   return lo;
 }
 
+// (calls of several windows only) The window's part of each class: its first
+// and last position by bisection, one lane each.
 __global__ void batch_window_begin_kernel(batch_job* job, uint32_t k) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  if (blockIdx.x != 0 || threadIdx.x >= 2 * kOpClasses) return;
   if (ld32_coherent(&job->bad)) return;
-  const unsigned long long first = job->first_op;
-  job->w_lo = (uint32_t)(job->offsets[window_start(job, k)] - first);
-  job->w_hi = (uint32_t)(job->offsets[window_start(job, k + 1)] - first);
-  job->n_writes = 0;
-  job->n_finds = 0;
-  job->n_ranges = 0;
-  job->n_epochs = 0;
+  const uint32_t q = threadIdx.x >> 1, at_end = threadIdx.x & 1;
+  const uint32_t target = (uint32_t)(job->offsets[window_start(job, k + at_end)] - job->first_op);
+  const uint32_t* part = job->list + (q > 1 ? job->total[1] : 0u);
+  uint32_t lo = 0, hi = job->total[q];  // the first entry of an operation >= target
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if ((q == 0 ? job->writes[mid].rel & 0x7FFFFFFFu : part[mid]) < target) lo = mid + 1;
+    else hi = mid;
+  }
+  const uint32_t other = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((threadIdx.x ^ 1u) << 2), (int)lo);
+  if (at_end) return;
+  job->first[q] = lo;
+  (q == 0 ? job->n_writes : q == 1 ? job->n_finds : job->n_ranges) = other - lo;
 }
 
 // End of a window: every read of the call at a snapshot below the next
@@ -777,84 +887,6 @@ __global__ void batch_window_end_kernel(batch_job* job, tree_state* st, epoch_st
   reclaim_prep(st, r ? ~0ull : 0ull, r ? series : nullptr);
 }
 
-// Operation classes of the split: writes (insert, erase), finds, ranges.
-MVBT_DEV uint32_t op_class(uint32_t ty) {
-  return (ty == kOpInsert || ty == kOpErase) ? 0u : ty == kOpFind ? 1u : ty == kOpRange ? 2u : 3u;
-}
-constexpr uint32_t kOpClasses = 3;
-
-// 6a. Operations of each class per segment (segments as in the sort):
-// seg[class * segments + segment]. A rejected call writes zero counts: the
-// scan and the radix passes that follow do not look at `bad`, and their
-// sizes come from these counts.
-__global__ void __launch_bounds__(kSortBlock) batch_split_count_kernel(batch_job* job) {
-  __shared__ uint32_t part[kOpClasses][kSortBlock / 64];
-  const uint32_t n = ld32_coherent(&job->bad) ? 0u : job->w_hi - job->w_lo;
-  const op_record* ops = job->ops + job->first_op + job->w_lo;
-  uint32_t a, b;
-  segment_of(n, blockIdx.x, gridDim.x, a, b);
-  uint32_t c[kOpClasses] = {0, 0, 0};
-  for (uint32_t i = a + threadIdx.x; i < b; i += kSortBlock) {
-    const uint32_t k = op_class(ops[i].type);
-#pragma unroll
-    for (uint32_t q = 0; q < kOpClasses; ++q) c[q] += k == q ? 1u : 0u;
-  }
-#pragma unroll
-  for (uint32_t q = 0; q < kOpClasses; ++q) {
-    for (int o = 32; o > 0; o >>= 1) c[q] += __shfl_xor(c[q], o, 64);
-    if ((threadIdx.x & 63) == 0) part[q][threadIdx.x >> 6] = c[q];
-  }
-  __syncthreads();
-  if (threadIdx.x < kOpClasses) {
-    uint32_t tot = 0;
-    for (uint32_t w = 0; w < kSortBlock / 64; ++w) tot += part[threadIdx.x][w];
-    job->seg[threadIdx.x * gridDim.x + blockIdx.x] = tot;
-  }
-}
-
-// 6b (after radix_scan_kernel turned the counts into offsets and the class
-// totals into n_writes, n_finds, n_ranges). Each class goes to its list in
-// operation order (a stable scatter per segment; no shared counter): writes
-// to w_rel, finds to rd_find, ranges to rd_range.
-__global__ void __launch_bounds__(kSortBlock) batch_split_kernel(batch_job* job) {
-  constexpr uint32_t kWaves = kSortBlock / 64;
-  __shared__ uint32_t wsum[kOpClasses][kWaves];
-  if (ld32_coherent(&job->bad)) return;
-  const uint32_t w_lo = job->w_lo, n = job->w_hi - w_lo;
-  const op_record* ops = job->ops + job->first_op + w_lo;
-  uint32_t* const lists[kOpClasses] = {job->w_rel, job->rd_find, job->rd_range};
-  const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6, G = gridDim.x;
-  const uint64_t below = (1ull << lane) - 1;
-  uint32_t a, b;
-  segment_of(n, blockIdx.x, G, a, b);
-  uint32_t run[kOpClasses];
-#pragma unroll
-  for (uint32_t q = 0; q < kOpClasses; ++q) run[q] = job->seg[q * G + blockIdx.x];
-  for (uint32_t c = a; c < b; c += kSortBlock) {
-    const uint32_t i = c + tid;
-    const uint32_t k = i < b ? op_class(ops[i].type) : 3u;
-    uint64_t m[kOpClasses];
-#pragma unroll
-    for (uint32_t q = 0; q < kOpClasses; ++q) {
-      m[q] = __builtin_amdgcn_ballot_w64(k == q);
-      if (lane == 0) wsum[q][w] = (uint32_t)__builtin_popcountll(m[q]);
-    }
-    __syncthreads();
-#pragma unroll
-    for (uint32_t q = 0; q < kOpClasses; ++q) {
-      uint32_t pos = run[q] + (uint32_t)__builtin_popcountll(m[q] & below), tot = 0;
-#pragma unroll
-      for (uint32_t v = 0; v < kWaves; ++v) {
-        if (v < w) pos += wsum[q][v];
-        tot += wsum[q][v];
-      }
-      if (k == q) lists[q][pos] = w_lo + i;
-      run[q] += tot;
-    }
-    __syncthreads();
-  }
-}
-
 // How the sorted form's kernels divide n operations, a count only the device
 // knows: one to a tile while that leaves tiles idle, then as few as keep
 // `tiles` of them busy (as split_for does for the plain launches).
@@ -863,9 +895,9 @@ MVBT_DEV uint32_t per_tile(uint32_t n, uint32_t tiles, uint32_t width) {
   return p < 1 ? 1u : p < width ? p : width;
 }
 
-// 7. Routes every write to its leaf: sort key = leaf (cap_ for a key that is
-// not routed: reserved keys, which fail in the write pass), payload = the
-// write's position in w_rel; the parent goes to w_par. T: routing tile
+// 7. Routes every write of the window to its leaf: sort key = leaf (cap_ for a
+// key that is not routed: reserved keys, which fail in the write pass), payload
+// = the write's position in the window; the parent goes to w_par. T: routing tile
 // width (T < NW: NW / T pairs per lane, mvbt_wide.hpp).
 template <int NW, int T = NW>
 __global__ void __launch_bounds__(256) batch_route_kernel(tree_ptrs tp, batch_job* job) {
@@ -877,15 +909,14 @@ __global__ void __launch_bounds__(256) batch_route_kernel(tree_ptrs tp, batch_jo
   if (c.block_ops(n) == 0) return;
   __shared__ route_cache<NW, kRangeCacheBytes> rc;
   tv.build_route_cache(rc, c.per >= kCachedFrom ? 0ull : ~0ull);
-  const op_record* ops = job->ops + job->first_op;
-  const uint32_t* w_rel = job->w_rel;
+  const write_rec* writes = job->writes + job->first[0];
   uint32_t* hint = job->sort_k[0];
   uint32_t* pos = job->sort_v[0];
   uint32_t* w_par = job->w_par;
   for (uint64_t base = c.first; base < n; base += c.stride) {
     const uint64_t i = base + t.rank();
     const bool act = c.holds(base, t.rank(), n);
-    const uint32_t key = act ? ops[w_rel[i]].key : 0u;
+    const uint32_t key = act ? writes[i].key : 0u;
     const bool go = act && valid_key(key);
     const uint64_t q = t.ballot(go);
     uint32_t st0 = kNone, sp0 = kNone, leaf = kNone, par = kNone;
@@ -903,33 +934,48 @@ __global__ void __launch_bounds__(256) batch_route_kernel(tree_ptrs tp, batch_jo
   }
 }
 
-// 7'. Copy planning. Every (leaf, batch) group of the sorted writes may copy
-// its leaf once, so the groups are counted and numbered here (a stable
-// count / scan / assign over the sorted list) and one reservation takes a
-// slot for each from the free stack and the never-used frontier, and enters
-// them all in the retire ring: the write pass then copies into its group's
-// slot without touching the shared allocation and retirement counters. A
-// slot its group does not use (no change, or the per-key path took over)
-// is simply freed by the next reclamation.
-MVBT_DEV bool epoch_start(const batch_job* job, const uint32_t* hint, const uint32_t* pos, uint32_t i) {
-  if (i == 0) return true;
-  if (hint[i] != hint[i - 1]) return true;
-  const uint32_t* op_batch = job->op_batch;
-  const uint32_t* w_rel = job->w_rel;
-  return op_batch[w_rel[pos[i]]] != op_batch[w_rel[pos[i - 1]]];
-}
-
-__global__ void __launch_bounds__(kSortBlock) batch_epoch_count_kernel(batch_job* job, uint32_t which) {
+// 7'. The sorted writes' fields in sorted order, so that the write pass reads
+// them with coalesced loads instead of chasing the position and the write one
+// dependent load after another, and the copy planning: every (leaf, batch)
+// group of the sorted writes may copy its leaf once, so the groups are counted
+// here and numbered below (a stable count / scan / assign over the sorted
+// list), and one reservation takes a slot for each from the free stack and the
+// never-used frontier, and enters them all in the retire ring: the write pass
+// then copies into its group's slot without touching the shared allocation and
+// retirement counters. A slot its group does not use (no change, or the
+// per-key path took over) is simply freed by the next reclamation.
+__global__ void __launch_bounds__(kSortBlock) batch_gather_kernel(batch_job* job, uint32_t which) {
   __shared__ uint32_t part[kSortBlock / 64];
   const uint32_t n = ld32_coherent(&job->bad) ? 0u : job->n_writes;
-  const uint32_t* hint = job->sort_k[which];
-  const uint32_t* pos = job->sort_v[which];
-  uint32_t a, b;
-  segment_of(n, blockIdx.x, gridDim.x, a, b);
-  uint32_t c = 0;
-  for (uint32_t i = a + threadIdx.x; i < b; i += kSortBlock) c += epoch_start(job, hint, pos, i) ? 1u : 0u;
+  const uint32_t *hint = job->sort_k[which], *pos = job->sort_v[which];
+  const write_rec* writes = job->writes + job->first[0];
+  const uint32_t lane = threadIdx.x & 63;
+  uint32_t a, e, c = 0;
+  segment_of(n, blockIdx.x, gridDim.x, a, e);
+  for (uint32_t i0 = a; i0 < e; i0 += kSortBlock) {
+    const uint32_t i = i0 + threadIdx.x;
+    const bool act = i < e;
+    uint32_t b = 0, h = 0;
+    if (act) {
+      const uint32_t p = pos[i];
+      h = hint[i];
+      const write_rec r = writes[p];
+      b = r.batch;
+      job->sorted[i] = r;
+      job->sort_k[which ^ 1u][i] = job->w_par[p];
+    }
+    // the write before this one in sorted order: the lane below, or a load
+    uint32_t hb = (uint32_t)__shfl_up((int)h, 1, 64), bb = (uint32_t)__shfl_up((int)b, 1, 64);
+    if (act && lane == 0 && i > 0) {
+      hb = hint[i - 1];
+      bb = writes[pos[i - 1]].batch;
+    }
+    const bool start = act && (i == 0 || h != hb || b != bb);
+    if (act) job->sort_v[which ^ 1u][i] = start ? 1u : 0u;  // read, then replaced, by batch_assign_kernel
+    c += start ? 1u : 0u;
+  }
   for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = c;
+  if (lane == 0) part[threadIdx.x >> 6] = c;
   __syncthreads();
   if (threadIdx.x == 0) {
     uint32_t tot = 0;
@@ -938,47 +984,17 @@ __global__ void __launch_bounds__(kSortBlock) batch_epoch_count_kernel(batch_job
   }
 }
 
-// (after radix_scan_kernel: seg holds each segment's first group number and
-// n_epochs the total) ep[i] = the group number of sorted write i.
-__global__ void __launch_bounds__(kSortBlock) batch_epoch_assign_kernel(batch_job* job, uint32_t which) {
-  constexpr uint32_t kWaves = kSortBlock / 64;
-  __shared__ uint32_t wsum[kWaves];
+// One workgroup: seg to each segment's first group number; its last thread,
+// which holds the number of groups, reserves a slot for each (free stack first,
+// then the frontier) and as many retire-ring positions as slots exist.
+__global__ void __launch_bounds__(kSortBlock)
+    batch_copy_reserve_kernel(batch_job* job, tree_ptrs tp, uint32_t segments) {
+  __shared__ scan_lds l;
   if (ld32_coherent(&job->bad)) return;
-  const uint32_t n = job->n_writes;
-  const uint32_t* hint = job->sort_k[which];
-  const uint32_t* pos = job->sort_v[which];
-  uint32_t* ep = job->sort_k[which ^ 1u];
-  const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const uint64_t below = (1ull << lane) - 1;
-  uint32_t a, b;
-  segment_of(n, blockIdx.x, gridDim.x, a, b);
-  uint32_t run = job->seg[blockIdx.x];  // groups started before this segment
-  for (uint32_t c = a; c < b; c += kSortBlock) {
-    const uint32_t i = c + tid;
-    const bool st = i < b && epoch_start(job, hint, pos, i);
-    const uint64_t m = __builtin_amdgcn_ballot_w64(st);
-    if (lane == 0) wsum[w] = (uint32_t)__builtin_popcountll(m);
-    __syncthreads();
-    uint32_t before = run + (uint32_t)__builtin_popcountll(m & below), tot = 0;
-#pragma unroll
-    for (uint32_t v = 0; v < kWaves; ++v) {
-      if (v < w) before += wsum[v];
-      tot += wsum[v];
-    }
-    // the group number is the count of starts at or before i, minus one
-    if (i < b) ep[i] = before + (st ? 1u : 0u) - 1u;
-    run += tot;
-    __syncthreads();
-  }
-}
-
-// One thread: reserves n_epochs slots (free stack first, then the
-// frontier) and as many retire-ring positions as slots exist.
-__global__ void batch_copy_reserve_kernel(batch_job* job, tree_ptrs tp) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (ld32_coherent(&job->bad)) return;
+  const uint32_t E = scan_row(job->seg, segments, l);
+  if (threadIdx.x != kSortBlock - 1) return;
+  job->n_epochs = E;
   tree_state* st = tp.st;
-  const uint32_t E = job->n_epochs;
   long long top = atomic_add_s64(&st->free_top, -(long long)E);
   const uint32_t got = (uint32_t)(top < 0 ? 0 : (top > (long long)E ? (long long)E : top));
   unsigned long long b = 0;
@@ -994,45 +1010,44 @@ __global__ void batch_copy_reserve_kernel(batch_job* job, tree_ptrs tp) {
   job->cp_ring = ring;
 }
 
-// Writes the slot of every group (kNone past the pool) to cslot and the
-// existing ones to the retire ring.
-__global__ void batch_copy_slots_kernel(batch_job* job, tree_ptrs tp, uint32_t which) {
+// The slot of every sorted write's group (kNone past the pool); the existing
+// ones go to the retire ring, each by its group's first write.
+__global__ void __launch_bounds__(kSortBlock) batch_assign_kernel(batch_job* job, tree_ptrs tp, uint32_t which) {
+  constexpr uint32_t kWaves = kSortBlock / 64;
+  __shared__ uint32_t wsum[kWaves];
   if (ld32_coherent(&job->bad)) return;
-  const uint32_t E = job->n_epochs, got = job->cp_got, valid = job->cp_valid;
+  const uint32_t n = job->n_writes, got = job->cp_got, valid = job->cp_valid;
   const long long top = job->cp_top;
-  const unsigned long long b = job->cp_bump, ring = job->cp_ring;
-  const unsigned long long mask = tp.retire_cap - 1;
-  uint32_t* cslot = job->sort_v[which ^ 1u];
-  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < E; k += gridDim.x * blockDim.x) {
-    uint32_t slot = kNone;
-    if (k < got) slot = ld32_coherent(tp.free_stack + (top - 1 - (long long)k));
-    else if (k < valid) slot = (uint32_t)(b + (k - got));
-    cslot[k] = slot;
-    if (k < valid) tp.retire_ring[(ring + k) & mask] = slot;
-  }
-}
-
-// 7''. Gathers each sorted write's fields into sorted order, so the write
-// pass reads them with coalesced loads instead of chasing the position, the
-// operation and its batch one dependent load after another.
-__global__ void __launch_bounds__(256) batch_gather_kernel(batch_job* job, uint32_t which) {
-  if (ld32_coherent(&job->bad)) return;
-  const uint32_t n = job->n_writes;
-  const uint32_t* pos = job->sort_v[which];
-  const uint32_t* ep = job->sort_k[which ^ 1u];
-  const uint32_t* cslot = job->sort_v[which ^ 1u];
-  const op_record* ops = job->ops + job->first_op;
-  uint32_t* const* g = job->gat;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const uint32_t pv = pos[i];
-    const uint32_t rel = job->w_rel[pv];
-    const op_record o = ops[rel];
-    g[0][i] = o.key;
-    g[1][i] = o.arg;
-    g[2][i] = rel | (o.type == kOpErase ? 0x80000000u : 0u);
-    g[3][i] = job->op_batch[rel];
-    g[4][i] = job->w_par[pv];
-    g[5][i] = cslot[ep[i]];
+  const unsigned long long bump = job->cp_bump, ring = job->cp_ring, mask = tp.retire_cap - 1;
+  uint32_t* slots = job->sort_v[which ^ 1u];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const uint64_t below = (1ull << lane) - 1;
+  uint32_t a, e;
+  segment_of(n, blockIdx.x, gridDim.x, a, e);
+  uint32_t run = job->seg[blockIdx.x];  // groups started before this segment
+  for (uint32_t c = a; c < e; c += kSortBlock) {
+    const uint32_t i = c + tid;
+    const bool act = i < e;
+    const bool start = act && slots[i] != 0;
+    const uint64_t m = __builtin_amdgcn_ballot_w64(start);
+    if (lane == 0) wsum[w] = (uint32_t)__builtin_popcountll(m);
+    __syncthreads();
+    uint32_t before = run + (uint32_t)__builtin_popcountll(m & below), tot = 0;
+#pragma unroll
+    for (uint32_t v = 0; v < kWaves; ++v) {
+      if (v < w) before += wsum[v];
+      tot += wsum[v];
+    }
+    if (act) {
+      const uint32_t k = before + (start ? 1u : 0u) - 1u;  // the write's group: starts at or before it, minus one
+      uint32_t slot = kNone;
+      if (k < got) slot = ld32_coherent(tp.free_stack + (top - 1 - (long long)k));
+      else if (k < valid) slot = (uint32_t)(bump + (k - got));
+      slots[i] = slot;
+      if (start && k < valid) tp.retire_ring[(ring + k) & mask] = slot;
+    }
+    run += tot;
+    __syncthreads();
   }
 }
 
@@ -1046,7 +1061,8 @@ __global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, b
   const uint32_t n = job->n_writes;
   const chunking<NW> c(per_tile(n, gridDim.x * (blockDim.x / NW), NW));
   const uint32_t* hint = job->sort_k[which];
-  const uint32_t* const* g = job->gat;  // the writes' fields in sorted order
+  const write_rec* recs = job->sorted;
+  const uint32_t *pars = job->sort_k[which ^ 1u], *slots = job->sort_v[which ^ 1u];
   uint32_t* results = job->results + job->first_op;
   const uint32_t clock0 = job->clock0;
   write_ctx ctx = tv.begin_writes(t);
@@ -1077,14 +1093,14 @@ __global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, b
       op_record op{};
       uint32_t rel = 0, b = 0, par = kNone, planned = kNone;
       if (act) {
-        op.key = g[0][i];
-        op.arg = g[1][i];
-        const uint32_t rt = g[2][i];
-        rel = rt & 0x7FFFFFFFu;
-        op.type = (rt >> 31) ? kOpErase : kOpInsert;
-        b = g[3][i];
-        par = g[4][i];
-        planned = g[5][i];
+        const write_rec w = recs[i];
+        op.key = w.key;
+        op.arg = w.arg;
+        rel = w.rel & 0x7FFFFFFFu;
+        op.type = (w.rel >> 31) ? kOpErase : kOpInsert;
+        b = w.batch;
+        par = pars[i];
+        planned = slots[i];
       }
       const uint32_t cur = clock0 + b + 1;
       const uint32_t leaf = (act && h < tv.cap_) ? h : kNone;
@@ -1140,7 +1156,7 @@ batch_sorted_find_kernel(tree_ptrs tp, const batch_job* job) {
   if (c.block_ops(n) == 0) return;
   __shared__ route_cache<NW, kFindCacheBytes> rc;
   tv.build_route_cache(rc, c.per >= kCachedFrom ? 0ull : ~0ull);
-  const uint32_t* list = job->rd_find;
+  const uint32_t* list = job->list + job->first[1];
   const uint32_t* op_batch = job->op_batch;
   const op_record* ops = job->ops + job->first_op;
   uint32_t* results = job->results + job->first_op;
@@ -1186,7 +1202,7 @@ __global__ void __launch_bounds__(256) batch_sorted_range_kernel(tree_ptrs tp, c
   if (c.block_ops(n) == 0) return;
   __shared__ rc_t rc;
   tv.build_route_cache(rc, c.per >= kCachedFrom ? 0ull : ~0ull);
-  const uint32_t* list = job->rd_range;
+  const uint32_t* list = job->list + job->total[1] + job->first[2];
   const uint32_t* op_batch = job->op_batch;
   const op_record* ops = job->ops + job->first_op;
   uint32_t* results = job->results + job->first_op;

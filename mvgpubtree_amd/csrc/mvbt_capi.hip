@@ -103,8 +103,8 @@ struct mvbt_tree {
   uint64_t b_hash_cap = 0;  // entries (a power of two)
   uint32_t* b_op_batch = nullptr;
   uint64_t b_op_cap = 0;    // entries
-  // sorted form (worker mode 2): 8 arrays of b_op_cap entries and the sort's
-  // segment counts and histograms, in one allocation
+  // sorted form (worker mode 2): kSortedArrays arrays of b_sorted_cap entries and
+  // the segment counts and histograms, in one allocation
   uint32_t* b_sorted = nullptr;
   uint64_t b_sorted_cap = 0;  // entries per array
   uint32_t worker_waves = 16;
@@ -634,10 +634,25 @@ constexpr uint64_t conflict_entries(uint64_t n) {
 }
 
 // Entries of the sorted form's allocation before its histograms.
-constexpr uint64_t kSortedArrays = 14;  // 8 working arrays + 6 gathered write fields
-constexpr uint64_t kSegWords = (uint64_t)kOpClasses * kSortSegments;  // the split's segment counts
+constexpr uint64_t kSortedArrays = 14;  // list .. sorted of batch_job (a write_rec array counts four)
+constexpr uint64_t kSegWords = (uint64_t)kOpClasses * kSliceWaves;  // the slices' class counts
+static_assert(kSliceBlocks <= kSegWords, "the copy planning's segment counts lie there too");
 constexpr uint64_t sorted_scratch_words(uint64_t cap) {
   return kSortedArrays * cap + kSegWords + (uint64_t)kRadix * kSortSegments + kRadix;
+}
+
+// The sorted form's pointers (batch_job list .. hist) into such an allocation of
+// `cap` entries an array.
+static_assert(offsetof(batch_job, hist) == offsetof(batch_job, list) + (kSortedPtrs - 1) * sizeof(void*),
+              "sorted scratch layout");
+void sorted_pointers(uint32_t* a, uint64_t cap, uint32_t** sp) {
+  const uint32_t words[] = {1, 4, 1, 1, 1, 1, 1, 4};  // list, writes, w_par, sort_k[2], sort_v[2], sorted
+  for (uint32_t k = 0; k < 8; ++k) {
+    sp[k] = a;
+    a += words[k] * cap;
+  }
+  sp[8] = a;              // seg
+  sp[9] = a + kSegWords;  // hist
 }
 
 // ---- allocation-free batched form (mvbt_run_batches_noalloc) ----------------
@@ -705,15 +720,9 @@ mvbt_status ensure_batch_scratch(mvbt_tree* t, uint32_t nb, uint64_t nops) {
     t->b_sorted_cap = 0;
     MVBT_HIP(hipMalloc(&t->b_sorted, sorted_scratch_words(cap) * sizeof(uint32_t)));
     t->b_sorted_cap = cap;
-    uint32_t* a = t->b_sorted;
-    // w_rel, w_par, sort_k[0..1], sort_v[0..1], rd_find, rd_range, seg, hist, gat[0..5]
-    uint32_t* sp[16];
-    for (uint64_t k = 0; k < 8; ++k) sp[k] = a + k * cap;
-    sp[8] = a + kSortedArrays * cap;
-    sp[9] = sp[8] + kSegWords;
-    for (uint64_t k = 0; k < 6; ++k) sp[10 + k] = a + (8 + k) * cap;
-    static_assert(offsetof(batch_job, gat) == offsetof(batch_job, w_rel) + 10 * sizeof(void*), "sorted scratch layout");
-    MVBT_HIP(hipMemcpy(&t->job->w_rel, sp, sizeof(sp), hipMemcpyHostToDevice));
+    uint32_t* sp[kSortedPtrs];
+    sorted_pointers(t->b_sorted, cap, sp);
+    MVBT_HIP(hipMemcpy(&t->job->list, sp, sizeof(sp), hipMemcpyHostToDevice));
     destroy_graph(t);  // the sort kernels of the graph take these pointers
   }
   if (nb <= t->b_capacity && want_hash <= t->b_hash_cap && nops <= t->b_op_cap) return MVBT_OK;
@@ -779,41 +788,26 @@ bool may_reclaim_in_call(const mvbt_tree* t, uint32_t flags) {
   return !(flags & MVBT_NO_RECLAIM) && t->live.empty() && !t->external_writers;
 }
 
-// Window k of the sorted form: begin, split, route, sort, copy planning,
-// write, find, range, end (reclamation when allowed, spill merge).
+// Window k of the sorted form: begin, route, sort, copy planning, write, find,
+// range, end (reclamation when allowed, spill merge).
 template <class Add>
-mvbt_status sorted_window(mvbt_tree* t, Add& add, batch_job* job, uint32_t* a, uint64_t cap, uint32_t k) {
-  uint32_t* sk[2] = {a + 2 * cap, a + 3 * cap};
-  {
+mvbt_status sorted_window(mvbt_tree* t, Add& add, batch_job* job, uint32_t* a, uint64_t cap, uint32_t k,
+                          uint32_t windows) {
+  uint32_t* sp[kSortedPtrs];
+  sorted_pointers(a, cap, sp);
+  uint32_t* sk[2] = {sp[3], sp[4]};
+  uint32_t* sv[2] = {sp[5], sp[6]};
+  if (windows > 1) {
     void* args[] = {&job, &k};
     if (hipError_t e = add(reinterpret_cast<void*>(&batch_window_begin_kernel), 1, 64, args)) return hip_fail(e);
   }
-  uint32_t* sv[2] = {a + 4 * cap, a + 5 * cap};
-  uint32_t* seg = a + kSortedArrays * cap;
-  uint32_t* hist = seg + kSegWords;
+  uint32_t* hist = sp[9];
   uint32_t* totals = hist + (uint64_t)kRadix * kSortSegments;
   uint32_t* n_writes = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(job) + offsetof(batch_job, n_writes));
-  uint32_t segs = kSortSegments;
+  uint32_t segs = kSortSegments, plan_segs = kSliceBlocks;
   const sorted_fns f = table_for(t->nw, true)->sorted(t->read_tile);
   tree_ptrs tp = t->ptrs();
   const uint32_t grid = (uint32_t)t->num_cus * 8;
-  {
-    void* args[] = {&job};
-    if (hipError_t e = add(reinterpret_cast<void*>(&batch_split_count_kernel), kSortSegments, kSortBlock, args))
-      return hip_fail(e);
-  }
-  {
-    // one row per operation class: totals land in n_writes, n_finds, n_ranges
-    static_assert(offsetof(batch_job, n_ranges) == offsetof(batch_job, n_writes) + 2 * sizeof(uint32_t), "counts");
-    void* args[] = {&seg, &segs, &n_writes};
-    if (hipError_t e = add(reinterpret_cast<void*>(&radix_scan_kernel), kOpClasses, kSortBlock, args))
-      return hip_fail(e);
-  }
-  {
-    void* args[] = {&job};
-    if (hipError_t e = add(reinterpret_cast<void*>(&batch_split_kernel), kSortSegments, kSortBlock, args))
-      return hip_fail(e);
-  }
   {
     void* args[] = {&tp, &job};
     if (hipError_t e = add(f.route, grid, kBlock, args)) return hip_fail(e);
@@ -837,21 +831,15 @@ mvbt_status sorted_window(mvbt_tree* t, Add& add, batch_job* job, uint32_t* a, u
   }
   uint32_t which = passes & 1;  // the buffer the last pass wrote
   {
-    // copy planning: number the (leaf, batch) groups, reserve a slot for each
-    uint32_t* n_epochs = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(job) + offsetof(batch_job, n_epochs));
+    // copy planning: count the (leaf, batch) groups, reserve a slot for each, hand them out
     void* args[] = {&job, &which};
-    if (hipError_t e = add(reinterpret_cast<void*>(&batch_epoch_count_kernel), kSortSegments, kSortBlock, args))
+    if (hipError_t e = add(reinterpret_cast<void*>(&batch_gather_kernel), plan_segs, kSortBlock, args))
       return hip_fail(e);
-    void* sargs[] = {&seg, &segs, &n_epochs};
-    if (hipError_t e = add(reinterpret_cast<void*>(&radix_scan_kernel), 1, kSortBlock, sargs)) return hip_fail(e);
-    if (hipError_t e = add(reinterpret_cast<void*>(&batch_epoch_assign_kernel), kSortSegments, kSortBlock, args))
+    void* rargs[] = {&job, &tp, &plan_segs};
+    if (hipError_t e = add(reinterpret_cast<void*>(&batch_copy_reserve_kernel), 1, kSortBlock, rargs)) return hip_fail(e);
+    void* sargs[] = {&job, &tp, &which};
+    if (hipError_t e = add(reinterpret_cast<void*>(&batch_assign_kernel), plan_segs, kSortBlock, sargs))
       return hip_fail(e);
-    void* rargs[] = {&job, &tp};
-    if (hipError_t e = add(reinterpret_cast<void*>(&batch_copy_reserve_kernel), 1, 64, rargs)) return hip_fail(e);
-    void* cargs[] = {&job, &tp, &which};
-    if (hipError_t e = add(reinterpret_cast<void*>(&batch_copy_slots_kernel), grid, kBlock, cargs))
-      return hip_fail(e);
-    if (hipError_t e = add(reinterpret_cast<void*>(&batch_gather_kernel), grid, kBlock, args)) return hip_fail(e);
   }
   {
     // the write pass's occupancy is the tunable one (worker waves per CU)
@@ -881,10 +869,20 @@ mvbt_status sorted_window(mvbt_tree* t, Add& add, batch_job* job, uint32_t* a, u
   return MVBT_OK;
 }
 
+// Everything after setup: the checks and the split by class, then the windows.
 template <class Add>
 mvbt_status sorted_sequence(mvbt_tree* t, Add&& add, batch_job* job, uint32_t* a, uint64_t cap, uint32_t windows) {
+  tree_state* st = t->st;
+  void* cargs[] = {&job, &st};
+  void* jargs[] = {&job};
+  if (hipError_t e = add(reinterpret_cast<void*>(&batch_slice_kernel), kSliceBlocks, kSortBlock, cargs)) return hip_fail(e);
+  if (hipError_t e = add(reinterpret_cast<void*>(&batch_class_scan_kernel), kOpClasses, kSortBlock, jargs))
+    return hip_fail(e);
+  if (hipError_t e = add(reinterpret_cast<void*>(&batch_split_kernel), kSliceBlocks, kSortBlock, jargs)) return hip_fail(e);
+  if (hipError_t e = add(reinterpret_cast<void*>(&batch_claim_kernel), (uint32_t)t->num_cus * 8, kSortBlock, cargs))
+    return hip_fail(e);
   for (uint32_t k = 0; k < windows; ++k)
-    if (mvbt_status rc = sorted_window(t, add, job, a, cap, k)) return rc;
+    if (mvbt_status rc = sorted_window(t, add, job, a, cap, k, windows)) return rc;
   return MVBT_OK;
 }
 
@@ -921,8 +919,8 @@ uint32_t effective_mode(const mvbt_tree* t, uint64_t num_ops) {
   return num_ops < kAutoSortedOps ? 0u : 2u;
 }
 
-// Explicit graph: setup -> count -> mask -> clear -> conflict -> (frontier -> worker | the sorted
-// form's windows) -> finish. Every node but setup reads its inputs from the
+// Explicit graph: setup -> (count -> mask -> clear -> conflict -> frontier -> worker | the sorted
+// form's checks and windows). Every node but setup reads its inputs from the
 // device descriptor, so a call only updates the setup node's parameters.
 mvbt_status build_graph(mvbt_tree* t, const batch_params& bp) {
   const uint32_t gi = graph_index(t, bp.windows);
@@ -948,21 +946,18 @@ mvbt_status build_graph(mvbt_tree* t, const batch_params& bp) {
   void* count_args[] = {&job, &st};
   MVBT_HIP(add(reinterpret_cast<void*>(&batch_setup_kernel), 1, 64, setup_args));
   t->graph_setup[gi] = node;
-  MVBT_HIP(add(t->eff_mode == 2 ? reinterpret_cast<void*>(&batch_slice_kernel)
-                                : reinterpret_cast<void*>(&batch_count_kernel),
-               t->num_cus * 4, kBlock, count_args));
-  MVBT_HIP(add(reinterpret_cast<void*>(&batch_mask_kernel), 1, 64, job_args));
-  MVBT_HIP(add(reinterpret_cast<void*>(&batch_clear_kernel), t->num_cus * 4, kBlock, job_args));
-  MVBT_HIP(add(reinterpret_cast<void*>(&batch_conflict_kernel), t->num_cus * 8, kBlock, count_args));
   if (t->eff_mode == 2) {
     if (mvbt_status rc = sorted_sequence(t, add, t->job, t->b_sorted, t->b_sorted_cap, bp.windows)) return rc;
   } else {
+    MVBT_HIP(add(reinterpret_cast<void*>(&batch_count_kernel), t->num_cus * 4, kBlock, count_args));
+    MVBT_HIP(add(reinterpret_cast<void*>(&batch_mask_kernel), 1, 64, job_args));
+    MVBT_HIP(add(reinterpret_cast<void*>(&batch_clear_kernel), t->num_cus * 4, kBlock, job_args));
+    MVBT_HIP(add(reinterpret_cast<void*>(&batch_conflict_kernel), t->num_cus * 8, kBlock, count_args));
     MVBT_HIP(add(reinterpret_cast<void*>(&batch_frontier_kernel), t->num_cus, kBlock, job_args));
     tree_ptrs tp = t->ptrs();
     void* worker_args[] = {&tp, &job};
     MVBT_HIP(add(worker_kernel(t), worker_blocks(t), kBlock, worker_args));
   }
-  MVBT_HIP(add(reinterpret_cast<void*>(&batch_finish_kernel), 1, 64, job_args));
   MVBT_HIP(hipGraphInstantiate(&t->graph_exec[gi], t->graph[gi], nullptr, nullptr, 0));
   return MVBT_OK;
 }
@@ -1518,19 +1513,16 @@ mvbt_status mvbt_run_batches(mvbt_tree* t, const mvbt_op* ops, uint64_t num_ops,
     MVBT_HIP(hipGraphLaunch(t->graph_exec[gi], s));
   } else {
     hipLaunchKernelGGL(batch_setup_kernel, dim3(1), dim3(64), 0, s, t->job, t->st, p);
-    if (t->eff_mode == 2)
-      hipLaunchKernelGGL(batch_slice_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job, t->st);
-    else
-      hipLaunchKernelGGL(batch_count_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job, t->st);
-    hipLaunchKernelGGL(batch_mask_kernel, dim3(1), dim3(64), 0, s, t->job);
-    hipLaunchKernelGGL(batch_clear_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job);
-    hipLaunchKernelGGL(batch_conflict_kernel, dim3(t->num_cus * 8), dim3(kBlock), 0, s, t->job, t->st);
     if (t->eff_mode == 2) {
       auto launch = [s](void* fn, unsigned grid, unsigned block, void** args) -> hipError_t {
         return hipLaunchKernel(fn, dim3(grid), dim3(block), args, 0, s);
       };
       if (mvbt_status rc = sorted_sequence(t, launch, t->job, t->b_sorted, t->b_sorted_cap, p.windows)) return rc;
     } else {
+      hipLaunchKernelGGL(batch_count_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job, t->st);
+      hipLaunchKernelGGL(batch_mask_kernel, dim3(1), dim3(64), 0, s, t->job);
+      hipLaunchKernelGGL(batch_clear_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job);
+      hipLaunchKernelGGL(batch_conflict_kernel, dim3(t->num_cus * 8), dim3(kBlock), 0, s, t->job, t->st);
       hipLaunchKernelGGL(batch_frontier_kernel, dim3(t->num_cus), dim3(kBlock), 0, s, t->job);
       tree_ptrs tp = t->ptrs();
       batch_job* job = t->job;
@@ -1538,7 +1530,6 @@ mvbt_status mvbt_run_batches(mvbt_tree* t, const mvbt_op* ops, uint64_t num_ops,
       MVBT_HIP(hipLaunchKernel(worker_kernel(t), dim3(worker_blocks(t)), dim3(kBlock),
                                wargs, 0, s));
     }
-    hipLaunchKernelGGL(batch_finish_kernel, dim3(1), dim3(64), 0, s, t->job);
   }
   MVBT_HIP(hipGetLastError());
   if (mvbt_status rc = clock_advanced(t, s, num_batches)) return rc;
@@ -1605,10 +1596,7 @@ mvbt_status mvbt_run_batches_noalloc(mvbt_tree* t, const mvbt_op* ops, uint64_t 
   l.hash = w + 3 * kNoAllocMaxBatches;
   l.op_batch = l.hash + kNoAllocHash;
   uint32_t* sorted = l.op_batch + kNoAllocMaxOps;
-  for (uint64_t k = 0; k < 8; ++k) l.sorted[k] = sorted + k * kNoAllocMaxOps;
-  l.sorted[8] = sorted + kSortedArrays * kNoAllocMaxOps;
-  l.sorted[9] = l.sorted[8] + kSegWords;
-  for (uint64_t k = 0; k < 6; ++k) l.sorted[10 + k] = sorted + (8 + k) * kNoAllocMaxOps;
+  sorted_pointers(sorted, kNoAllocMaxOps, l.sorted);
   batch_params p{};
   p.ops = reinterpret_cast<const op_record*>(ops);
   p.nops = num_ops;
@@ -1626,15 +1614,10 @@ mvbt_status mvbt_run_batches_noalloc(mvbt_tree* t, const mvbt_op* ops, uint64_t 
   p.reclaim = may_reclaim_in_call(t, 0) ? 1u : 0u;
   hipLaunchKernelGGL(batch_bind_kernel, dim3(1), dim3(64), 0, s, job, l);
   hipLaunchKernelGGL(batch_setup_kernel, dim3(1), dim3(64), 0, s, job, t->st, p);
-  hipLaunchKernelGGL(batch_slice_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, job, t->st);
-  hipLaunchKernelGGL(batch_mask_kernel, dim3(1), dim3(64), 0, s, job);
-  hipLaunchKernelGGL(batch_clear_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, job);
-  hipLaunchKernelGGL(batch_conflict_kernel, dim3(t->num_cus * 8), dim3(kBlock), 0, s, job, t->st);
   auto launch = [s](void* fn, unsigned grid, unsigned block, void** args) -> hipError_t {
     return hipLaunchKernel(fn, dim3(grid), dim3(block), args, 0, s);
   };
   if (mvbt_status rc = sorted_sequence(t, launch, job, sorted, kNoAllocMaxOps, p.windows)) return rc;
-  hipLaunchKernelGGL(batch_finish_kernel, dim3(1), dim3(64), 0, s, job);
   MVBT_HIP(hipGetLastError());
   if (mvbt_status rc = clock_advanced(t, s, num_batches)) return rc;
   if (mvbt_status rc = isolated_done(t, s)) return rc;

@@ -48,31 +48,47 @@ __global__ void __launch_bounds__(kSortBlock)
   hist[tid * gridDim.x + blockIdx.x] = h[tid];
 }
 
+// Exclusive scan of a row of at most kScanMax in place by one workgroup, read
+// and written coalesced through LDS (one word of padding a bank row); returns
+// the row's total on its last thread.
+constexpr uint32_t kScanMax = 4096;
+struct scan_lds {
+  uint32_t part[kSortBlock];
+  uint32_t row[kScanMax + kScanMax / 32];
+};
+MVBT_DEV uint32_t scan_row(uint32_t* row, uint32_t n, scan_lds& l) {
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t i = tid; i < n; i += kSortBlock) l.row[i + i / 32] = row[i];
+  __syncthreads();
+  const uint32_t per = (n + kSortBlock - 1) / kSortBlock;
+  const uint32_t a = tid * per, b = a + per < n ? a + per : n;
+  uint32_t s = 0;
+  for (uint32_t i = a; i < b; ++i) s += l.row[i + i / 32];
+  l.part[tid] = s;
+  __syncthreads();
+  for (uint32_t off = 1; off < kSortBlock; off <<= 1) {  // inclusive scan (Hillis-Steele)
+    const uint32_t v = tid >= off ? l.part[tid - off] : 0u;
+    __syncthreads();
+    l.part[tid] += v;
+    __syncthreads();
+  }
+  uint32_t run = l.part[tid] - s;  // exclusive
+  for (uint32_t i = a; i < b; ++i) {
+    const uint32_t c = l.row[i + i / 32];
+    l.row[i + i / 32] = run;
+    run += c;
+  }
+  __syncthreads();
+  for (uint32_t i = tid; i < n; i += kSortBlock) row[i] = l.row[i + i / 32];
+  return l.part[tid];
+}
+
 // One workgroup per digit (gridDim.x = 256), G = `segments` counts each.
 __global__ void __launch_bounds__(kSortBlock)
     radix_scan_kernel(uint32_t* hist, uint32_t segments, uint32_t* totals) {
-  __shared__ uint32_t part[kSortBlock];
-  const uint32_t tid = threadIdx.x, d = blockIdx.x;
-  uint32_t* row = hist + (size_t)d * segments;
-  const uint32_t per = (segments + kSortBlock - 1) / kSortBlock;
-  const uint32_t a = tid * per, b = a + per < segments ? a + per : segments;
-  uint32_t s = 0;
-  for (uint32_t i = a; i < b; ++i) s += row[i];
-  part[tid] = s;
-  __syncthreads();
-  for (uint32_t off = 1; off < kSortBlock; off <<= 1) {  // inclusive scan (Hillis-Steele)
-    const uint32_t v = tid >= off ? part[tid - off] : 0u;
-    __syncthreads();
-    part[tid] += v;
-    __syncthreads();
-  }
-  uint32_t run = part[tid] - s;  // exclusive
-  for (uint32_t i = a; i < b; ++i) {
-    const uint32_t c = row[i];
-    row[i] = run;
-    run += c;
-  }
-  if (tid == kSortBlock - 1) totals[d] = part[tid];
+  __shared__ scan_lds l;
+  const uint32_t total = scan_row(hist + (size_t)blockIdx.x * segments, segments, l);
+  if (threadIdx.x == kSortBlock - 1) totals[blockIdx.x] = total;
 }
 
 __global__ void __launch_bounds__(kSortBlock)
