@@ -276,7 +276,7 @@ typedef struct mvbt_op {
  * btree_kernels.hpp:31-306) to any mix, deterministically. Runs num_batches batches in
  * one launch sequence (a persistent work-queue worker in worker modes 0 and 1; the
  * sorted form in mode 2: every write grouped by leaf and applied in batch order, then
- * every read at its batch's snapshot; mode 3, the default, picks by call size, see
+ * every read at its batch's snapshot; mode 3, the default, is the sorted form too, see
  * mvbt_set_worker_mode). batch_offsets (device, num_batches + 1 entries) are
  * absolute indices into ops: batch b is ops[offsets[b] .. offsets[b+1]), results go to
  * the same indices (so `results` must cover index offsets[num_batches] - 1), and
@@ -315,8 +315,8 @@ mvbt_status mvbt_run_batches(mvbt_tree* tree, const mvbt_op* ops, uint64_t num_o
 
 /* No counterpart in the reference (a capacity hint, like std::vector::reserve): sizes
  * the batched form's scratch for calls of up to num_ops operations and num_batches
- * batches and builds the launch graphs of the current worker mode (in mode 3, of both
- * forms a call of that size or smaller may run in), so that later such calls allocate
+ * batches and builds the launch graphs of the current worker mode (in modes 2 and 3, of
+ * every form a call of that size or smaller may run in), so that later such calls allocate
  * nothing and build nothing. Synchronous. */
 mvbt_status mvbt_reserve_batches(mvbt_tree* tree, uint64_t num_ops, uint32_t num_batches);
 
@@ -353,9 +353,9 @@ mvbt_status mvbt_set_worker_waves(mvbt_tree* tree, uint32_t waves_per_cu);
  * writes of the per-batch kernels; 2 = the sorted form: the call's writes are routed
  * to their leaves, sorted by leaf (stable radix sort), and applied leaf group by leaf
  * group in batch order by the tile that owns the group, then every find and range runs
- * at its batch's snapshot in one pass; 3 (default) = by call size: mode 0 for calls of
- * fewer than 16384 operations (the sorted form's launch sequence then costs more than
- * it saves), mode 2 from there up. Same results in every mode. */
+ * at its batch's snapshot in one pass; 3 (default) = mode 2, except that calls of
+ * fewer than 16384 operations keep their version copies until mvbt_reclaim. Same
+ * results in every mode. */
 mvbt_status mvbt_set_worker_mode(mvbt_tree* tree, uint32_t mode);
 
 /* Read tile width (autotuner knob; the reference's tile is always its node width,

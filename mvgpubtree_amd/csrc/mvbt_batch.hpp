@@ -1051,6 +1051,294 @@ __global__ void __launch_bounds__(kSortBlock) batch_assign_kernel(batch_job* job
   }
 }
 
+// ---- small calls of the sorted form ----------------------------------------
+// A call of at most kSmallOps operations in at most kSmallBatches batches: a
+// launch costs 4-5 us whatever it does, and the 24 of a window are most of such
+// a call (3000 operations: 146 us on the batch-after-batch worker, no less in
+// the launches above). One workgroup therefore does the checks and the split,
+// and after the routing one workgroup sorts the writes in LDS and plans their
+// copies: the call is 8 launches.
+constexpr uint32_t kSmallOps = 16384, kSmallBatches = 4096, kSmallBlock = 1024;
+
+// Exclusive prefix of `v` over the workgroup's threads; *total: its sum. `w`:
+// kSmallBlock / 64 words of LDS.
+MVBT_DEV uint32_t block_prefix(uint32_t v, uint32_t* w, uint32_t* total) {
+  constexpr uint32_t kWaves = kSmallBlock / 64;
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t incl = v;
+#pragma unroll
+  for (uint32_t d = 1; d < 64; d <<= 1) {
+    const uint32_t up = (uint32_t)__shfl_up((int)incl, (int)d, 64);
+    if (lane >= d) incl += up;
+  }
+  if (lane == 63) w[wave] = incl;
+  __syncthreads();
+  uint32_t before = 0, all = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kWaves; ++k) {
+    if (k < wave) before += w[k];
+    all += w[k];
+  }
+  __syncthreads();
+  *total = all;
+  return before + incl - v;
+}
+
+// S1. Setup, batches, checks and split of a small call, by one workgroup.
+__global__ void __launch_bounds__(kSmallBlock) batch_small_begin_kernel(batch_job* job, tree_state* st, batch_params p) {
+  constexpr uint32_t kWaves = kSmallBlock / 64;
+  __shared__ uint32_t table[2 * kSmallOps];
+  __shared__ uint32_t off[kSmallBatches + 1];
+  __shared__ uint32_t wsum[kOpClasses][kWaves];
+  __shared__ uint32_t bad;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nb = p.nb, n = (uint32_t)p.nops;
+  const unsigned long long first = p.offsets[0];
+  if (tid == 0) bad = p.offsets[nb] - first == p.nops ? 0u : 1u;  // (last < first differs as well)
+  __syncthreads();
+  for (uint32_t b = tid; b <= nb; b += kSmallBlock) {
+    const unsigned long long o = p.offsets[b] - first;
+    if (o > n || (b > 0 && p.offsets[b] < p.offsets[b - 1])) bad = 1;
+    off[b] = (uint32_t)o;
+  }
+  __syncthreads();
+  const bool ordered = bad == 0;
+  uint32_t run[kOpClasses] = {0, 0, 0};
+  const op_record* ops = p.ops + first;
+  const uint64_t below = (1ull << lane) - 1;
+  // finds and ranges share `list`: the ranges go in behind n - 1 downwards and are turned round below
+  for (uint32_t i0 = 0; ordered && i0 < n; i0 += kSmallBlock) {
+    const uint32_t i = i0 + tid;
+    op_record o{};
+    uint32_t k = kOpClasses, b = 0;
+    if (i < n) {
+      o = ops[i];
+      uint32_t hi = nb;
+      while (hi - b > 1) {  // off[b] <= i < off[hi]
+        const uint32_t mid = (b + hi) >> 1;
+        if (off[mid] <= i) b = mid;
+        else hi = mid;
+      }
+      job->op_batch[i] = b;
+      k = op_class(o.type);
+      if (k == kOpClasses) bad = 1;
+    }
+    uint64_t m[kOpClasses];
+#pragma unroll
+    for (uint32_t q = 0; q < kOpClasses; ++q) {
+      m[q] = __builtin_amdgcn_ballot_w64(k == q);
+      if (lane == 0) wsum[q][w] = (uint32_t)__builtin_popcountll(m[q]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t q = 0; q < kOpClasses; ++q) {
+      uint32_t pos = run[q] + (uint32_t)__builtin_popcountll(m[q] & below), tot = 0;
+#pragma unroll
+      for (uint32_t v = 0; v < kWaves; ++v) {
+        if (v < w) pos += wsum[q][v];
+        tot += wsum[q][v];
+      }
+      if (k == q) {
+        if (q == 0) job->writes[pos] = write_rec{o.key, o.arg, i | (o.type == kOpErase ? 0x80000000u : 0u), b};
+        else job->list[q == 1 ? pos : n - 1 - pos] = i;
+      }
+      run[q] += tot;
+    }
+    __syncthreads();
+  }
+  // distinct write keys per batch (as batch_claim_kernel, with the table in LDS)
+  uint32_t mask = 1023;
+  while (mask + 1 < 2 * run[0]) mask = 2 * mask + 1;
+  for (uint32_t i = tid; i <= mask; i += kSmallBlock) table[i] = 0;
+  __syncthreads();
+  for (uint32_t i = tid; i < run[0]; i += kSmallBlock) {
+    const write_rec r = job->writes[i];
+    if (!valid_key(r.key)) continue;
+    uint32_t h = conflict_hash(r.key, r.batch) & mask;
+    for (uint32_t probe = 0; probe <= mask; ++probe) {
+      const uint32_t cur = atomicCAS(&table[h], 0u, i + 1);
+      if (cur == 0) break;
+      if (job->writes[cur - 1].key == r.key && job->writes[cur - 1].batch == r.batch) {
+        bad = 1;
+        break;
+      }
+      h = (h + 1) & mask;
+    }
+  }
+  // the ranges, turned round, behind the finds (each pair of entries by one thread)
+  __syncthreads();
+  const uint32_t nf = run[1], nr = run[2];
+  uint32_t mine[(kSmallOps + kSmallBlock - 1) / kSmallBlock];
+#pragma unroll
+  for (uint32_t j = 0; j < (kSmallOps + kSmallBlock - 1) / kSmallBlock; ++j) {
+    const uint32_t r = tid + j * kSmallBlock;
+    if (r < nr) mine[j] = job->list[n - 1 - r];
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t j = 0; j < (kSmallOps + kSmallBlock - 1) / kSmallBlock; ++j) {
+    const uint32_t r = tid + j * kSmallBlock;
+    if (r < nr) job->list[nf + r] = mine[j];
+  }
+  if (tid == 0) {
+    const uint32_t clock0 = __hip_atomic_fetch_add(&st->clock, nb, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    if (p.base_out) *p.base_out = clock0;
+    job->ops = p.ops;
+    job->offsets = p.offsets;
+    job->nb = nb;
+    job->L = p.L;
+    job->results = p.results;
+    job->pairs = p.pairs;
+    job->pair_slots = p.pair_slots;
+    job->clock0 = clock0;
+    job->first_op = first;
+    job->nops = ordered ? first + n : first;
+    job->bad = bad;
+    job->windows = 1;
+    job->reclaim = p.reclaim;
+    for (uint32_t q = 0; q < kOpClasses; ++q) {
+      job->first[q] = 0;
+      job->total[q] = run[q];
+    }
+    job->n_writes = run[0];
+    job->n_finds = nf;
+    job->n_ranges = nr;
+    if (bad) atomic_or32(&st->error_flags, kErrBadBatch);
+  }
+}
+
+// S2. Sort by leaf, gather and copy planning of a small call's writes, by one
+// workgroup: three 8-bit radix passes (bits covers the pool's indices) with
+// leaf and position in LDS, each wave ranking its own stretch; then what
+// batch_gather_kernel, batch_copy_reserve_kernel and batch_assign_kernel do.
+// The sorted leaf hints end in sort_k[1], as after an odd number of passes.
+__global__ void __launch_bounds__(kSmallBlock) batch_small_plan_kernel(batch_job* job, tree_ptrs tp, uint32_t bits) {
+  constexpr uint32_t kWaves = kSmallBlock / 64, kItems = kSmallOps / kSmallBlock;
+  __shared__ uint32_t key[kSmallOps];
+  __shared__ uint16_t pos[kSmallOps];
+  __shared__ uint16_t bat[kSmallOps];
+  __shared__ uint32_t cnt[kWaves][kRadix];
+  __shared__ uint32_t wsum[kWaves];
+  __shared__ long long s_top;
+  __shared__ unsigned long long s_bump, s_ring;
+  __shared__ uint32_t s_got, s_valid;
+  if (ld32_coherent(&job->bad)) return;
+  const uint32_t n = job->n_writes;
+  if (n == 0) return;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const uint64_t below = (1ull << lane) - 1;
+  const write_rec* writes = job->writes;
+  for (uint32_t i = tid; i < n; i += kSmallBlock) {
+    key[i] = job->sort_k[0][i];
+    pos[i] = (uint16_t)i;
+  }
+  __syncthreads();
+  // wave w ranks items [w * S, (w + 1) * S), 64 at a time
+  const uint32_t S = ((n + kWaves - 1) / kWaves + 63) / 64 * 64, a = w * S;
+  for (uint32_t shift = 0; shift < bits; shift += 8) {
+    volatile uint32_t* my = cnt[w];  // this wave's alone until the barrier; its LDS operations run in order
+    for (uint32_t d = lane; d < kRadix; d += 64) my[d] = 0;
+    uint32_t k[kItems], v[kItems], rank[kItems];
+#pragma unroll
+    for (uint32_t j = 0; j < kItems; ++j) {
+      const uint32_t i = a + j * 64 + lane;
+      const bool act = j * 64 < S && i < n;
+      if (__builtin_amdgcn_ballot_w64(act) == 0) continue;
+      k[j] = act ? key[i] : 0u;
+      v[j] = act ? pos[i] : 0u;
+      const uint32_t d = (k[j] >> shift) & (kRadix - 1);
+      uint64_t same = __builtin_amdgcn_ballot_w64(act);
+#pragma unroll
+      for (uint32_t bit = 0; bit < 8; ++bit) {
+        const uint64_t ones = __builtin_amdgcn_ballot_w64(((d >> bit) & 1u) != 0);
+        same &= ((d >> bit) & 1u) ? ones : ~ones;
+      }
+      const uint32_t before = my[d];  // this wave's earlier items with the digit
+      rank[j] = before + (uint32_t)__builtin_popcountll(same & below);
+      if (act && (same & below) == 0) my[d] = before + (uint32_t)__builtin_popcountll(same);
+    }
+    __syncthreads();
+    {  // exclusive prefix over (digit, wave): thread t holds waves 4 (t & 3) .. of digit t / 4
+      const uint32_t d = tid >> 2, w0 = (tid & 3) * (kWaves / 4);
+      uint32_t c[kWaves / 4], s = 0, total;
+#pragma unroll
+      for (uint32_t q = 0; q < kWaves / 4; ++q) {
+        c[q] = cnt[w0 + q][d];
+        s += c[q];
+      }
+      uint32_t r = block_prefix(s, wsum, &total);
+#pragma unroll
+      for (uint32_t q = 0; q < kWaves / 4; ++q) {
+        cnt[w0 + q][d] = r;
+        r += c[q];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < kItems; ++j) {
+      const uint32_t i = a + j * 64 + lane;
+      if (j * 64 < S && i < n) {
+        const uint32_t to = cnt[w][(k[j] >> shift) & (kRadix - 1)] + rank[j];
+        key[to] = k[j];
+        pos[to] = (uint16_t)v[j];
+      }
+    }
+    __syncthreads();
+  }
+  // sorted position i: the write's record and parent, and its batch
+  for (uint32_t i = tid; i < n; i += kSmallBlock) {
+    const write_rec r = writes[pos[i]];
+    job->sorted[i] = r;
+    bat[i] = (uint16_t)r.batch;
+    job->sort_k[1][i] = key[i];
+    job->sort_k[0][i] = job->w_par[pos[i]];
+  }
+  __syncthreads();
+  // groups started at or before each position; the slots are reserved in between
+  uint32_t group[kItems], run = 0;
+  bool start[kItems];
+#pragma unroll
+  for (uint32_t j = 0; j < kItems; ++j) {
+    if (j * kSmallBlock >= n) continue;
+    const uint32_t i = j * kSmallBlock + tid;
+    start[j] = i < n && (i == 0 || key[i] != key[i - 1] || bat[i] != bat[i - 1]);
+    uint32_t total;
+    group[j] = run + block_prefix(start[j] ? 1u : 0u, wsum, &total) + (start[j] ? 1u : 0u) - 1u;
+    run += total;
+  }
+  if (tid == 0) {
+    // all of them, or none where the pool has fewer left: the write pass then
+    // takes slots for the copies it does make, as a batch-by-batch call would
+    tree_state* st = tp.st;
+    const long long on_stack = (long long)ld_coherent((const uint64_t*)&st->free_top);
+    const unsigned long long used = ld_coherent((const uint64_t*)&st->bump);
+    const unsigned long long left = (used < tp.cap_ ? tp.cap_ - used : 0ull) + (on_stack > 0 ? (unsigned long long)on_stack : 0ull);
+    const uint32_t E = left < run ? 0u : run;
+    job->n_epochs = E;
+    s_got = s_valid = 0;
+    if (E) {
+      const long long top = atomic_add_s64(&st->free_top, -(long long)E);
+      const uint32_t got = (uint32_t)(top < 0 ? 0 : (top > (long long)E ? (long long)E : top));
+      s_top = top;
+      s_got = got;
+      if (got < E) s_bump = atomic_add64(&st->bump, (unsigned long long)(E - got));
+      s_valid = E;  // no other writer runs beside the call: what was left is still there
+      s_ring = atomic_add64(&st->retire_tail, (unsigned long long)E);
+    }
+  }
+  __syncthreads();
+  const unsigned long long mask = tp.retire_cap - 1;
+#pragma unroll
+  for (uint32_t j = 0; j < kItems; ++j) {
+    const uint32_t i = j * kSmallBlock + tid;
+    if (i >= n) continue;
+    uint32_t slot = kNone;
+    if (group[j] < s_got) slot = ld32_coherent(tp.free_stack + (s_top - 1 - (long long)group[j]));
+    else if (group[j] < s_valid) slot = (uint32_t)(s_bump + (group[j] - s_got));
+    job->sort_v[0][i] = slot;
+    if (start[j] && group[j] < s_valid) tp.retire_ring[(s_ring + group[j]) & mask] = slot;
+  }
+}
+
 // 8. The write pass over the sorted writes (buffers sort_k/v[which]).
 template <int NW>
 __global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, batch_job* job, uint32_t which) {

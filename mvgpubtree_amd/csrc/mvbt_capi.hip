@@ -110,15 +110,19 @@ struct mvbt_tree {
   uint32_t worker_waves = 16;
   // 0: one operation per tile; 1: chunks (batch_chunk_worker_kernel);
   // 2: sorted (writes grouped by leaf, then every read at its snapshot);
-  // 3: by call size (the persistent worker below kAutoSortedOps operations,
-  // the sorted form from there up). eff_mode: the mode of the current call.
+  // 3: as 2. eff_mode: the mode of the current call (kSmallSorted: a small
+  // call of the sorted form).
   uint32_t worker_mode = 3;
+  static constexpr uint32_t kSmallSorted = 4;
   uint32_t eff_mode = 2;
-  // launch graphs: [0] for worker modes 0 and 1, [k] for the sorted form in k windows
+  bool sorted_form() const { return eff_mode == 2 || eff_mode == kSmallSorted; }
+  // launch graphs: [0] for worker modes 0 and 1, [k] for the sorted form in k windows,
+  // [kMaxWindows + 1] for its small calls
   static constexpr uint32_t kMaxWindows = 16;
-  hipGraph_t graph[kMaxWindows + 1] = {};
-  hipGraphExec_t graph_exec[kMaxWindows + 1] = {};
-  hipGraphNode_t graph_setup[kMaxWindows + 1] = {};
+  static constexpr uint32_t kGraphs = kMaxWindows + 2;
+  hipGraph_t graph[kGraphs] = {};
+  hipGraphExec_t graph_exec[kGraphs] = {};
+  hipGraphNode_t graph_setup[kGraphs] = {};
   uint64_t window_ops = 1ull << 22;  // sorted form: operations per window (0: one window)
   // lanes per read tile of the launches in which no writer runs (finds and
   // ranges without MVBT_CONCURRENT, the sorted form's read passes); below the
@@ -707,7 +711,7 @@ mvbt_status ensure_batch_scratch(mvbt_tree* t, uint32_t nb, uint64_t nops) {
     MVBT_HIP(hipMemset(t->job, 0, sizeof(batch_job)));
   }
   const uint64_t want_hash = conflict_entries(nops);
-  const bool sorted = t->eff_mode == 2;
+  const bool sorted = t->sorted_form();
   if (nb <= t->b_capacity && want_hash <= t->b_hash_cap && nops <= t->b_op_cap &&
       (!sorted || nops <= t->b_sorted_cap))
     return MVBT_OK;
@@ -788,6 +792,9 @@ bool may_reclaim_in_call(const mvbt_tree* t, uint32_t flags) {
   return !(flags & MVBT_NO_RECLAIM) && t->live.empty() && !t->external_writers;
 }
 
+template <class Add>
+mvbt_status sorted_tail(mvbt_tree* t, Add& add, batch_job* job, uint32_t which);
+
 // Window k of the sorted form: begin, route, sort, copy planning, write, find,
 // range, end (reclamation when allowed, spill merge).
 template <class Add>
@@ -841,6 +848,15 @@ mvbt_status sorted_window(mvbt_tree* t, Add& add, batch_job* job, uint32_t* a, u
     if (hipError_t e = add(reinterpret_cast<void*>(&batch_assign_kernel), plan_segs, kSortBlock, sargs))
       return hip_fail(e);
   }
+  return sorted_tail(t, add, job, which);
+}
+
+// The write pass over the sorted writes (buffers sort_k/v[which]), the reads, and the end of a window.
+template <class Add>
+mvbt_status sorted_tail(mvbt_tree* t, Add& add, batch_job* job, uint32_t which) {
+  const sorted_fns f = table_for(t->nw, true)->sorted(t->read_tile);
+  tree_ptrs tp = t->ptrs();
+  const uint32_t grid = (uint32_t)t->num_cus * 8;
   {
     // the write pass's occupancy is the tunable one (worker waves per CU)
     void* args[] = {&tp, &job, &which};
@@ -886,13 +902,26 @@ mvbt_status sorted_sequence(mvbt_tree* t, Add&& add, batch_job* job, uint32_t* a
   return MVBT_OK;
 }
 
+// A small call after batch_small_begin_kernel: route, sort and plan, then as any window.
+template <class Add>
+mvbt_status small_sequence(mvbt_tree* t, Add&& add, batch_job* job) {
+  const sorted_fns f = table_for(t->nw, true)->sorted(t->read_tile);
+  tree_ptrs tp = t->ptrs();
+  uint32_t bits = 8 * sort_passes(t);
+  void* rargs[] = {&tp, &job};
+  if (hipError_t e = add(f.route, (uint32_t)t->num_cus * 8, kBlock, rargs)) return hip_fail(e);
+  void* pargs[] = {&job, &tp, &bits};
+  if (hipError_t e = add(reinterpret_cast<void*>(&batch_small_plan_kernel), 1, kSmallBlock, pargs)) return hip_fail(e);
+  return sorted_tail(t, add, job, 1);
+}
+
 void* worker_kernel(const mvbt_tree* t) {
   const dispatch_table* tb = table_for(t->nw, true);
   return t->eff_mode == 1 ? tb->chunk_worker() : tb->worker();
 }
 
 void destroy_graph(mvbt_tree* t) {
-  for (uint32_t g = 0; g <= mvbt_tree::kMaxWindows; ++g) {
+  for (uint32_t g = 0; g < mvbt_tree::kGraphs; ++g) {
     if (t->graph_exec[g]) (void)hipGraphExecDestroy(t->graph_exec[g]);
     if (t->graph[g]) (void)hipGraphDestroy(t->graph[g]);
     t->graph_exec[g] = nullptr;
@@ -908,15 +937,24 @@ uint32_t windows_for(const mvbt_tree* t, uint64_t num_ops, uint32_t num_batches)
   const uint64_t k = (num_ops + t->window_ops - 1) / t->window_ops;
   return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>({k, num_batches, mvbt_tree::kMaxWindows}));
 }
-uint32_t graph_index(const mvbt_tree* t, uint32_t windows) { return t->eff_mode == 2 ? windows : 0; }
+uint32_t graph_index(const mvbt_tree* t, uint32_t windows) {
+  return t->eff_mode == 2 ? windows : t->eff_mode == mvbt_tree::kSmallSorted ? mvbt_tree::kMaxWindows + 1 : 0;
+}
 
-// Below this many operations a call in mode 3 runs on the one-operation-per-
-// tile worker: the sorted form's 25-odd launches per window then cost more
-// than the frontier waits they save (served steps of one or two requests).
+// The form of a call. Modes 2 and 3 both run the sorted form, small calls of one
+// window in the form made for them. Mode 3 once ran calls below kAutoSortedOps
+// operations on the persistent worker, whose batches wait for each other: 146 us
+// for 3 batches of 3000 operations against 93 now, 422 against 145 for 24 of
+// 16384. Such calls still keep their version copies until mvbt_reclaim.
 constexpr uint64_t kAutoSortedOps = 16384;
-uint32_t effective_mode(const mvbt_tree* t, uint64_t num_ops) {
-  if (t->worker_mode != 3) return t->worker_mode;
-  return num_ops < kAutoSortedOps ? 0u : 2u;
+bool keeps_copies(const mvbt_tree* t, uint64_t num_ops) { return t->worker_mode == 3 && num_ops < kAutoSortedOps; }
+bool small_call(const mvbt_tree* t, uint64_t num_ops, uint32_t num_batches) {
+  return num_ops <= kSmallOps && num_batches <= kSmallBatches &&
+         (t->window_ops == 0 || num_ops <= t->window_ops || keeps_copies(t, num_ops));
+}
+uint32_t effective_mode(const mvbt_tree* t, uint64_t num_ops, uint32_t num_batches) {
+  if (t->worker_mode < 2) return t->worker_mode;
+  return small_call(t, num_ops, num_batches) ? mvbt_tree::kSmallSorted : 2u;
 }
 
 // Explicit graph: setup -> (count -> mask -> clear -> conflict -> frontier -> worker | the sorted
@@ -944,9 +982,13 @@ mvbt_status build_graph(mvbt_tree* t, const batch_params& bp) {
     return e;
   };
   void* count_args[] = {&job, &st};
-  MVBT_HIP(add(reinterpret_cast<void*>(&batch_setup_kernel), 1, 64, setup_args));
+  const bool small = t->eff_mode == mvbt_tree::kSmallSorted;
+  if (small) MVBT_HIP(add(reinterpret_cast<void*>(&batch_small_begin_kernel), 1, kSmallBlock, setup_args));
+  else MVBT_HIP(add(reinterpret_cast<void*>(&batch_setup_kernel), 1, 64, setup_args));
   t->graph_setup[gi] = node;
-  if (t->eff_mode == 2) {
+  if (small) {
+    if (mvbt_status rc = small_sequence(t, add, t->job)) return rc;
+  } else if (t->eff_mode == 2) {
     if (mvbt_status rc = sorted_sequence(t, add, t->job, t->b_sorted, t->b_sorted_cap, bp.windows)) return rc;
   } else {
     MVBT_HIP(add(reinterpret_cast<void*>(&batch_count_kernel), t->num_cus * 4, kBlock, count_args));
@@ -1477,7 +1519,7 @@ mvbt_status mvbt_run_batches(mvbt_tree* t, const mvbt_op* ops, uint64_t num_ops,
   if (pairs && L == 0) return fail(MVBT_ERR_INVALID_ARG, "L must be > 0 when pairs is given");
   device_guard g(t->device);
   std::lock_guard<std::mutex> lk(t->mu);
-  t->eff_mode = effective_mode(t, num_ops);
+  t->eff_mode = effective_mode(t, num_ops, num_batches);
   if (mvbt_status rc = reserve_ids(t, num_batches)) return rc;
   if (mvbt_status rc = ensure_batch_scratch(t, num_batches, num_ops)) return rc;
   hipStream_t s = (hipStream_t)stream;
@@ -1495,7 +1537,7 @@ mvbt_status mvbt_run_batches(mvbt_tree* t, const mvbt_op* ops, uint64_t num_ops,
   p.base_out = snapshot_base;
   p.hash_mask = (uint32_t)(conflict_entries(num_ops) - 1);
   p.windows = windows_for(t, num_ops, num_batches);
-  p.reclaim = may_reclaim_in_call(t, flags) ? 1u : 0u;
+  p.reclaim = may_reclaim_in_call(t, flags) && !keeps_copies(t, num_ops) ? 1u : 0u;
   if (flags & MVBT_USE_GRAPH) {
     const uint32_t gi = graph_index(t, p.windows);
     if (!t->graph_exec[gi]) {
@@ -1504,31 +1546,36 @@ mvbt_status mvbt_run_batches(mvbt_tree* t, const mvbt_op* ops, uint64_t num_ops,
     batch_job* job = t->job;
     tree_state* st = t->st;
     void* args[] = {&job, &st, &p};
+    const bool small = t->eff_mode == mvbt_tree::kSmallSorted;
     hipKernelNodeParams kp{};
-    kp.func = reinterpret_cast<void*>(&batch_setup_kernel);
+    kp.func = small ? reinterpret_cast<void*>(&batch_small_begin_kernel) : reinterpret_cast<void*>(&batch_setup_kernel);
     kp.gridDim = dim3(1);
-    kp.blockDim = dim3(64);
+    kp.blockDim = dim3(small ? kSmallBlock : 64);
     kp.kernelParams = args;
     MVBT_HIP(hipGraphExecKernelNodeSetParams(t->graph_exec[gi], t->graph_setup[gi], &kp));
     MVBT_HIP(hipGraphLaunch(t->graph_exec[gi], s));
   } else {
-    hipLaunchKernelGGL(batch_setup_kernel, dim3(1), dim3(64), 0, s, t->job, t->st, p);
-    if (t->eff_mode == 2) {
-      auto launch = [s](void* fn, unsigned grid, unsigned block, void** args) -> hipError_t {
-        return hipLaunchKernel(fn, dim3(grid), dim3(block), args, 0, s);
-      };
-      if (mvbt_status rc = sorted_sequence(t, launch, t->job, t->b_sorted, t->b_sorted_cap, p.windows)) return rc;
+    auto launch = [s](void* fn, unsigned grid, unsigned block, void** args) -> hipError_t {
+      return hipLaunchKernel(fn, dim3(grid), dim3(block), args, 0, s);
+    };
+    if (t->eff_mode == mvbt_tree::kSmallSorted) {
+      hipLaunchKernelGGL(batch_small_begin_kernel, dim3(1), dim3(kSmallBlock), 0, s, t->job, t->st, p);
+      if (mvbt_status rc = small_sequence(t, launch, t->job)) return rc;
     } else {
-      hipLaunchKernelGGL(batch_count_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job, t->st);
-      hipLaunchKernelGGL(batch_mask_kernel, dim3(1), dim3(64), 0, s, t->job);
-      hipLaunchKernelGGL(batch_clear_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job);
-      hipLaunchKernelGGL(batch_conflict_kernel, dim3(t->num_cus * 8), dim3(kBlock), 0, s, t->job, t->st);
-      hipLaunchKernelGGL(batch_frontier_kernel, dim3(t->num_cus), dim3(kBlock), 0, s, t->job);
-      tree_ptrs tp = t->ptrs();
-      batch_job* job = t->job;
-      void* wargs[] = {&tp, &job};
-      MVBT_HIP(hipLaunchKernel(worker_kernel(t), dim3(worker_blocks(t)), dim3(kBlock),
-                               wargs, 0, s));
+      hipLaunchKernelGGL(batch_setup_kernel, dim3(1), dim3(64), 0, s, t->job, t->st, p);
+      if (t->eff_mode == 2) {
+        if (mvbt_status rc = sorted_sequence(t, launch, t->job, t->b_sorted, t->b_sorted_cap, p.windows)) return rc;
+      } else {
+        hipLaunchKernelGGL(batch_count_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job, t->st);
+        hipLaunchKernelGGL(batch_mask_kernel, dim3(1), dim3(64), 0, s, t->job);
+        hipLaunchKernelGGL(batch_clear_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->job);
+        hipLaunchKernelGGL(batch_conflict_kernel, dim3(t->num_cus * 8), dim3(kBlock), 0, s, t->job, t->st);
+        hipLaunchKernelGGL(batch_frontier_kernel, dim3(t->num_cus), dim3(kBlock), 0, s, t->job);
+        tree_ptrs tp = t->ptrs();
+        batch_job* job = t->job;
+        void* wargs[] = {&tp, &job};
+        MVBT_HIP(hipLaunchKernel(worker_kernel(t), dim3(worker_blocks(t)), dim3(kBlock), wargs, 0, s));
+      }
     }
   }
   MVBT_HIP(hipGetLastError());
@@ -1544,9 +1591,9 @@ mvbt_status mvbt_reserve_batches(mvbt_tree* t, uint64_t num_ops, uint32_t num_ba
   if (num_ops >= (1ull << 31)) return fail(MVBT_ERR_INVALID_ARG, "num_ops must be below 2^31");
   device_guard g(t->device);
   std::lock_guard<std::mutex> lk(t->mu);
-  // every mode calls of up to num_ops operations may run in (both, in mode 3)
-  std::vector<uint32_t> modes{effective_mode(t, num_ops)};
-  if (t->worker_mode == 3 && num_ops >= kAutoSortedOps) modes.push_back(0);
+  // every form calls of up to that size may run in
+  std::vector<uint32_t> modes{effective_mode(t, num_ops, num_batches)};
+  if (modes[0] == 2) modes.push_back(mvbt_tree::kSmallSorted);
   for (uint32_t m : modes) {
     t->eff_mode = m;
     if (mvbt_status rc = ensure_batch_scratch(t, std::max<uint32_t>(num_batches, 1), std::max<uint64_t>(num_ops, 1)))
@@ -1613,11 +1660,16 @@ mvbt_status mvbt_run_batches_noalloc(mvbt_tree* t, const mvbt_op* ops, uint64_t 
       {(num_ops + t->window_ops - 1) / t->window_ops, num_batches, mvbt_tree::kMaxWindows}));
   p.reclaim = may_reclaim_in_call(t, 0) ? 1u : 0u;
   hipLaunchKernelGGL(batch_bind_kernel, dim3(1), dim3(64), 0, s, job, l);
-  hipLaunchKernelGGL(batch_setup_kernel, dim3(1), dim3(64), 0, s, job, t->st, p);
   auto launch = [s](void* fn, unsigned grid, unsigned block, void** args) -> hipError_t {
     return hipLaunchKernel(fn, dim3(grid), dim3(block), args, 0, s);
   };
-  if (mvbt_status rc = sorted_sequence(t, launch, job, sorted, kNoAllocMaxOps, p.windows)) return rc;
+  if (num_ops <= kSmallOps && num_batches <= kSmallBatches && p.windows == 1) {
+    hipLaunchKernelGGL(batch_small_begin_kernel, dim3(1), dim3(kSmallBlock), 0, s, job, t->st, p);
+    if (mvbt_status rc = small_sequence(t, launch, job)) return rc;
+  } else {
+    hipLaunchKernelGGL(batch_setup_kernel, dim3(1), dim3(64), 0, s, job, t->st, p);
+    if (mvbt_status rc = sorted_sequence(t, launch, job, sorted, kNoAllocMaxOps, p.windows)) return rc;
+  }
   MVBT_HIP(hipGetLastError());
   if (mvbt_status rc = clock_advanced(t, s, num_batches)) return rc;
   if (mvbt_status rc = isolated_done(t, s)) return rc;

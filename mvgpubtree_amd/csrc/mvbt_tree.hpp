@@ -1430,7 +1430,8 @@ struct tree_view : tree_ptrs {
   // PLANNED: `planned` (per lane, equal for the lanes of one leaf) is the
   // version-copy slot reserved for the leaf's epoch ahead of the launch and
   // already entered in the retire ring, so no copy allocates or retires here
-  // (kNone: the pool had no slot for it). PLANNED also takes no leaf locks:
+  // (kNone: none was reserved, and the tile allocates if the leaf needs it).
+  // PLANNED also takes no leaf locks:
   // in the sorted form's write pass every leaf has one writing tile (the one
   // that owns its group of sorted writes; a split's new right node holds
   // only keys of that group) and no reader runs, while the per-key path and
@@ -1545,9 +1546,10 @@ struct tree_view : tree_ptrs {
 #pragma unroll
           for (int i = 0; i < LB; ++i) {
             if (!((need_copy >> i) & 1)) continue;
-            const uint32_t slot = PLANNED ? t.shfl(planned, gl[i]) : alloc(c, t, true);
-            if (slot == kNone) {  // pool exhausted: leave the leaf unchanged
-              if (PLANNED) flag(kErrPoolExhausted, t);
+            uint32_t slot = PLANNED ? t.shfl(planned, gl[i]) : kNone;
+            const bool own = slot == kNone;
+            if (own) slot = alloc(c, t, true);
+            if (slot == kNone) {  // pool exhausted (flagged): leave the leaf unchanged
               ok &= ~(1u << i);
               changed &= ~(1u << i);
               need_copy &= ~(1u << i);
@@ -1556,7 +1558,7 @@ struct tree_view : tree_ptrs {
             node_t n;
             n.p = img[i];
             n.store_unlocked_copy(at(slot), t);
-            if (!PLANNED) retire(c, slot, t);
+            if (own) retire(c, slot, t);
             if (r == gl[i]) cp = slot;
           }
           if (need_copy) {
