@@ -974,11 +974,16 @@ struct tree_view : tree_ptrs {
           continue;
         }
       } else {
-        uint32_t l = 0;  // last entry whose pivot is <= key (entry 0 routes from the node's low bound)
+        // An entry whose pivot is <= key (entry 0 routes from the node's low
+        // bound), by halving steps: the last one in a whole image. In a torn
+        // one entry l still has a pivot <= key (or is entry 0), so its child
+        // lies at or left of the right one. Five dependent LDS reads a level
+        // instead of 29 that the LDS serves one wave after another.
+        uint32_t l = 0;
 #pragma unroll
-        for (uint32_t e = 1; e < node_t::kData; ++e) {
-          const uint32_t k = lo32(img[e]);
-          if (k != kEmpty && key >= k) l = e;
+        for (uint32_t step = NW / 2; step != 0; step >>= 1) {
+          const uint32_t e = l + step;
+          if (e < node_t::kData && lo32(img[e]) <= key) l = e;  // an empty entry's key is above every key
         }
         next = hi32(img[l]);
         parent = rc.index[s];
