@@ -1456,22 +1456,18 @@ batch_sorted_find_kernel(tree_ptrs tp, const batch_job* job) {
     const uint32_t key = act ? ops[rel].key : 0u;
     const uint32_t ts = act ? clock0 + op_batch[rel] : 0u;
     uint32_t result = kEmpty;
-    if constexpr (T < NW) {
+    if constexpr (T == 16) {
+      const bool go = act && valid_key(key);
+      uint32_t start = tv.root_, unused;
+      if (go) start = tv.route_lane(rc, key, unused);
+      result = find_rows(tv, key, ts, start, (uint32_t)t.ballot(go), c.per);
+    } else if constexpr (T < NW) {
       result = read_chunk_wide<T, false, true, kWideFindGroup<NW / T>>(tv, key, 0u, ts, nullptr, 0u, t.ballot(act), t,
                                                                         &rc);
     } else if constexpr (NW >= 32) {
       // as in find_kernel: the pass-based engine keeps more walks in flight
       result = tv.template read_chunk<false, route_cache<NW, kFindCacheBytes>, true, tree_view<NW, true>::kFindGroup>(
           key, 0u, ts, nullptr, 0u, t.ballot(act), t, &rc);
-    } else {
-      uint32_t start = kNone, unused;
-      if (act && valid_key(key)) start = tv.route_lane(rc, key, unused);
-      for (uint64_t q = t.ballot(act); q;) {
-        const uint32_t j = (uint32_t)lowest_bit(q);
-        q &= q - 1;
-        const uint32_t v = tv.template find<false>(t.shfl(key, j), t.shfl(ts, j), t, t.shfl(start, j));
-        if (t.rank() == j) result = v;
-      }
     }
     if (act) results[rel] = result;
   }
@@ -1510,13 +1506,18 @@ __global__ void __launch_bounds__(256) batch_sorted_range_kernel(tree_ptrs tp, c
       if (op.slot < pair_slots) out = pairs + (size_t)op.slot * L;
       else bad_slot = true;
     }
+    const uint32_t k0 = op.key == 0 ? 1u : op.key;
     uint32_t cnt;
-    if constexpr (T < NW)
-      cnt = read_chunk_wide<T, true, true, kWideRangeGroup<NW / T>>(tv, op.key == 0 ? 1u : op.key, op.arg, ts, out, L,
-                                                                    t.ballot(act), t, &rc);
-    else
-      cnt = tv.template read_chunk<true, rc_t, true>(op.key == 0 ? 1u : op.key, op.arg, ts, out, L, t.ballot(act), t,
-                                                     &rc);
+    if constexpr (T == 16) {
+      const bool go = act && valid_key(k0) && op.arg > k0;
+      uint32_t start = tv.root_, unused;
+      if (go) start = tv.route_lane(rc, k0, unused);
+      cnt = range_rows(tv, k0, op.arg, ts, start, out, L, (uint32_t)t.ballot(go));
+    } else if constexpr (T < NW) {
+      cnt = read_chunk_wide<T, true, true, kWideRangeGroup<NW / T>>(tv, k0, op.arg, ts, out, L, t.ballot(act), t, &rc);
+    } else {
+      cnt = tv.template read_chunk<true, rc_t, true>(k0, op.arg, ts, out, L, t.ballot(act), t, &rc);
+    }
     if (act) results[rel] = cnt;
     overflow |= act && cnt > L;
   }

@@ -187,7 +187,11 @@ work_split split_for(const mvbt_tree* t, uint64_t n, uint32_t width, int waves) 
   ws.cached = ws.per_tile >= kCachedFrom ? 1u : 0u;
   return ws;
 }
-constexpr int kFindWaves = 32, kRangeWaves = 16;  // about what the kernels hold of each CU
+// About what the kernels hold of each CU: ranges 32 waves with the 16-lane
+// quiescent reader (200K ranges of 32 pairs at 20M keys 101 us when divided for
+// 16, 80 for 32), 16 with the pass-based ones.
+constexpr int kFindWaves = 32;
+constexpr int range_waves(uint32_t width, bool conc) { return width == 16 && !conc ? 32 : 16; }
 
 // The same for write and mixed launches: a power of two (so a chunk lies in
 // one aligned group of `width` operations, see superseded()), for 12 waves on
@@ -259,7 +263,7 @@ struct impl {
                            uint32_t* counts, uint32_t L, uint64_t n, uint32_t ts, hipStream_t s,
                            bool conc) {
     const uint32_t width = !conc && t->read_tile ? t->read_tile : NW;
-    const work_split ws = split_for(t, n, width, kRangeWaves);
+    const work_split ws = split_for(t, n, width, range_waves(width, conc));
     if (!conc && (range_wide<16>(t, lo, hi, out, counts, L, n, ts, s, ws) ||
                   range_wide<32>(t, lo, hi, out, counts, L, n, ts, s, ws))) {
       MVBT_HIP(hipGetLastError());

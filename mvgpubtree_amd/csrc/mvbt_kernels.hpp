@@ -5,6 +5,7 @@
 // warp-cooperative work sharing (btree_kernels.hpp:507-517). Chunks are taken
 // grid-stride so a launch can be sized to residency instead of to n.
 #pragma once
+#include "mvbt_reads.hpp"
 #include "mvbt_tree.hpp"
 #include "mvbt_wide.hpp"
 
@@ -77,8 +78,9 @@ __global__ void init_kernel(tree_view<NW, VER> tv) {
 }
 
 // Finds and ranges with read tiles of T < NW lanes (P = NW / T pairs per
-// lane, mvbt_wide.hpp), for launches in which no writer runs: the same
-// pass-based reader, with 64 / T walks per wave. Walks advanced per pass:
+// lane), for launches in which no writer runs: 16-lane tiles through read_rows
+// (mvbt_reads.hpp), wider ones through the pass-based reader (mvbt_wide.hpp),
+// with 64 / T walks per wave. Walks advanced per pass:
 // kWideFindGroup at the find kernel's 8 waves per SIMD, kWideRangeGroup in
 // the range kernel (whose occupancy is not pinned).
 template <int P>
@@ -210,7 +212,12 @@ find_kernel(tree_view<NW, VER> tv, const uint32_t* keys,
     uint32_t key = active ? keys[i] : 0u;
     uint32_t result = kEmpty;
     uint64_t q = t.ballot(active);
-    if constexpr (!CONC && NW >= 32) {
+    if constexpr (!CONC && NW == 16) {
+      const bool go = active && valid_key(key);
+      uint32_t start = tv.root_, unused;
+      if (go) start = tv.route_lane(rc, key, unused);
+      result = find_rows(tv, key, ts, start, (uint32_t)t.ballot(go), c.per);
+    } else if constexpr (!CONC && NW >= 32) {
       // 32- and 64-pair tiles: a wave holds only two (one) of them, so one
       // walk per tile leaves too few loads in flight; the pass-based engine
       // advances kReadGroup walks of the tile per pass instead.
@@ -249,7 +256,13 @@ __global__ void __launch_bounds__(256)
     uint32_t hi = active ? upper[i] : 0u;
     uint32_t result = 0;
     uint64_t q = t.ballot(active);
-    if constexpr (!CONC) {
+    if constexpr (!CONC && NW == 16) {
+      const uint32_t k0 = lo == 0 ? 1u : lo;
+      const bool go = active && valid_key(k0) && hi > k0;
+      uint32_t start = tv.root_, unused;
+      if (go) start = tv.route_lane(rc, k0, unused);
+      result = range_rows(tv, k0, hi, ts, start, out ? out + i * (uint64_t)L : nullptr, L, (uint32_t)t.ballot(go));
+    } else if constexpr (!CONC) {
       // no writer runs: every query of the chunk advances one node per pass
       result = tv.template read_chunk<true>(lo == 0 ? 1u : lo, hi, ts, out ? out + base * (uint64_t)L : nullptr,
                                             L, q, t, &rc);
@@ -310,8 +323,16 @@ find_wide_kernel(tree_view<NW, VER> tv, const uint32_t* keys, uint32_t* values, 
     const uint64_t i = base + t.rank();
     const bool active = c.holds(base, t.rank(), n);
     const uint32_t key = active ? keys[i] : 0u;
-    const uint32_t result =
-        read_chunk_wide<T, false, false, kWideFindGroup<NW / T>>(tv, key, 0u, ts, nullptr, 0u, t.ballot(active), t, &rc);
+    uint32_t result;
+    if constexpr (T == 16) {
+      const bool go = active && valid_key(key);
+      uint32_t start = tv.root_, unused;
+      if (go) start = tv.route_lane(rc, key, unused);
+      result = find_rows(tv, key, ts, start, (uint32_t)t.ballot(go), c.per);
+    } else {
+      result = read_chunk_wide<T, false, false, kWideFindGroup<NW / T>>(tv, key, 0u, ts, nullptr, 0u, t.ballot(active),
+                                                                        t, &rc);
+    }
     if (active) values[i] = result;
   }
 }
@@ -330,8 +351,17 @@ __global__ void __launch_bounds__(256)
     const bool active = c.holds(base, t.rank(), n);
     const uint32_t lo = active ? lower[i] : 0u;
     const uint32_t hi = active ? upper[i] : 0u;
-    const uint32_t result = read_chunk_wide<T, true, false, kWideRangeGroup<NW / T>>(
-        tv, lo == 0 ? 1u : lo, hi, ts, out ? out + base * (uint64_t)L : nullptr, L, t.ballot(active), t, &rc);
+    const uint32_t k0 = lo == 0 ? 1u : lo;
+    uint32_t result;
+    if constexpr (T == 16) {
+      const bool go = active && valid_key(k0) && hi > k0;
+      uint32_t start = tv.root_, unused;
+      if (go) start = tv.route_lane(rc, k0, unused);
+      result = range_rows(tv, k0, hi, ts, start, out ? out + i * (uint64_t)L : nullptr, L, (uint32_t)t.ballot(go));
+    } else {
+      result = read_chunk_wide<T, true, false, kWideRangeGroup<NW / T>>(
+          tv, k0, hi, ts, out ? out + base * (uint64_t)L : nullptr, L, t.ballot(active), t, &rc);
+    }
     if (active && counts) counts[i] = result;
     if (t.any(active && result > L) && t.leader()) atomic_or32(&tv.st->error_flags, kErrRangeOverflow);
   }
