@@ -146,10 +146,34 @@ struct tile {
   MVBT_DEV uint64_t shfl64(uint64_t v, uint32_t src) const {
     return pack(shfl(lo32(v), src), shfl(hi32(v), src));
   }
-  // Value from lane rank-d (own value for rank < d).
-  MVBT_DEV uint64_t shfl_up64(uint64_t v, uint32_t d) const {
-    uint32_t r = rank();
-    return shfl64(v, r >= d ? r - d : r);
+  // Lane SRC's value on every lane of the tile, without the LDS permute's trip:
+  // a DPP row broadcast (a row is 16 lanes), then for 32 lanes the odd and even
+  // rows exchanged (permlane16_swap(x, x) leaves every even row's x in its
+  // first result and every odd row's in its second).
+  template <uint32_t SRC>
+  MVBT_DEV uint32_t bcast(uint32_t v) const {
+    static_assert(SRC < (uint32_t)W, "a lane of the tile");
+    if constexpr (W == 64) {
+      return (uint32_t)__builtin_amdgcn_readlane((int)v, SRC);
+    } else {
+      const uint32_t x = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 | (SRC & 15), 0xf, 0xf, true);
+      if constexpr (W == 16) return x;
+      const auto both = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+      return SRC < 16 ? both[0] : both[1];
+    }
+  }
+  template <uint32_t SRC>
+  MVBT_DEV uint64_t bcast64(uint64_t v) const {
+    return pack(bcast<SRC>(lo32(v)), bcast<SRC>(hi32(v)));
+  }
+  // Value from the lane below (above); undefined on the tile's first (last) lane.
+  MVBT_DEV uint64_t from_below(uint64_t v) const {
+    return pack((uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo32(v), 0x138, 0xf, 0xf, true),
+                (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi32(v), 0x138, 0xf, 0xf, true));
+  }
+  MVBT_DEV uint64_t from_above(uint64_t v) const {
+    return pack((uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo32(v), 0x130, 0xf, 0xf, true),
+                (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi32(v), 0x130, 0xf, 0xf, true));
   }
   // Value from lane rank+d (own value past the end).
   MVBT_DEV uint64_t shfl_down64(uint64_t v, uint32_t d) const {
@@ -157,6 +181,14 @@ struct tile {
     return shfl64(v, r + d < (uint32_t)W ? r + d : r);
   }
 };
+
+// The same value, which the compiler takes for a new one: what is derived from
+// it is computed again where it is used instead of being kept in registers.
+template <class V>
+MVBT_DEV V again(V v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
 
 MVBT_DEV int highest_bit(uint64_t m) { return m ? 63 - __builtin_clzll(m) : -1; }
 MVBT_DEV int lowest_bit(uint64_t m) { return m ? __builtin_ctzll(m) : -1; }

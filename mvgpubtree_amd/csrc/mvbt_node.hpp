@@ -55,8 +55,8 @@ struct node {
 
   // ---- metadata -----------------------------------------------------------
   MVBT_DEV uint64_t lane_pair(uint32_t r, const tile_t& t) const { return t.shfl64(p, r); }
-  MVBT_DEV uint64_t meta(const tile_t& t) const { return lane_pair(kMetaLane, t); }
-  MVBT_DEV uint64_t version(const tile_t& t) const { return lane_pair(kVerLane, t); }
+  MVBT_DEV uint64_t meta(const tile_t& t) const { return t.template bcast64<kMetaLane>(p); }
+  MVBT_DEV uint64_t version(const tile_t& t) const { return t.template bcast64<kVerLane>(p); }
   MVBT_DEV static uint32_t high_key(uint64_t meta) { return lo32(meta); }
   MVBT_DEV static uint32_t sibling(uint64_t meta) { return hi32(meta) & kPtrMask; }
   MVBT_DEV static bool is_leaf(uint64_t meta) { return (hi32(meta) & kLeafBit) != 0; }
@@ -122,7 +122,7 @@ struct node {
     }
     uint64_t gt = t.ballot(data_lane(r) && this->key() != kEmpty && key > this->key());
     uint32_t pos = (uint32_t)(highest_bit(gt) + 1);
-    uint64_t up = t.shfl_up64(p, 1);
+    uint64_t up = t.from_below(p);  // (lane 0 never takes it: its r > pos fails)
     if (data_lane(r)) {
       if (r == pos) p = pack(key, value);
       else if (r > pos) p = up;
@@ -135,7 +135,7 @@ struct node {
     uint64_t eq = t.ballot(data_lane(r) && this->key() == key);
     if (!eq) return false;
     uint32_t pos = (uint32_t)lowest_bit(eq);
-    uint64_t down = t.shfl_down64(p, 1);
+    uint64_t down = t.from_above(p);  // (the last data lane does not take it)
     if (data_lane(r) && r >= pos) p = (r == kLastData) ? kEmptyPair : down;
     return true;
   }
@@ -156,7 +156,7 @@ struct node {
 
   // ---- split ----------------------------------------------------------------
   // Pivot = first key of the upper half.
-  MVBT_DEV uint32_t split_pivot(const tile_t& t) const { return lo32(lane_pair(kHalf, t)); }
+  MVBT_DEV uint32_t split_pivot(const tile_t& t) const { return t.template bcast<kHalf>(lo32(p)); }
 
   // Upper half of this node as a new right sibling (data lanes shifted down
   // by kHalf); its metadata inherits this node's high key and sibling.

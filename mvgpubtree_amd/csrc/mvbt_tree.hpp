@@ -1408,22 +1408,28 @@ struct tree_view : tree_ptrs {
   // Batched leaf phase for a routed chunk (lane j: key j, value j, routed
   // leaf j; `q` the keys to write). Every leaf that receives the chunk's keys
   // is locked at once (one lane-parallel atomic). The locked leaves are then
-  // handled kLeafBatch at a time, each step for all of them before the next:
-  // reload, apply the keys in registers in lane order, store the version
-  // copies, one wait, store the version words (lane-parallel), one wait,
-  // store the data lanes; the next batch's reloads are issued before the wait
-  // that completes those stores, and then this batch is unlocked
-  // (lane-parallel). Per leaf this is the order write() uses (copy -> version
-  // word -> data -> unlock), so snapshot readers validate the same way; a
-  // chunk pays about three waits per batch of leaves instead of six per key.
+  // handled kLeafBatch at a time: reload them all, wait; apply each leaf's keys
+  // in registers in lane order and store its version copy; wait; store the
+  // version words (lane-parallel); wait; store the data lanes; the next
+  // batch's reloads are issued before the wait that completes those stores,
+  // and then this batch is unlocked (lane-parallel). Per leaf this is the
+  // order write() uses (copy -> version word -> data -> unlock), so snapshot
+  // readers validate the same way; a chunk pays about three waits per batch of
+  // leaves instead of six per key.
   // No lock is waited for here and every lock is released before returning,
   // so the tiles of a wave never wait on each other's locks inside it. Keys
   // whose leaf was not locked, would overflow, or no longer covers the key
   // are returned as a mask for write(); lane j's `result` receives
   // kWriteNew / kWriteSame for the others.
-  // 32-pair nodes take 32-key chunks: batches of 12 leaves cover them in
-  // three rounds within the same register budget (4 waves per SIMD).
-  static constexpr int kLeafBatch = NW == 32 ? 12 : 8;
+  // What bounds it: random accesses of whole nodes (one pass of 500K random
+  // 256-byte nodes on MI355X: loads 56 us, stores 28, the lock atomics 42), of
+  // which each key costs a load, two stores and two words here. The reloads are
+  // waited for all at once: loads and stores share one counter, so with copies
+  // going out between the uses of the loads every use also waits for the
+  // copies before it (500K inserts at 40M keys, 32 pairs: 309 us; with the one
+  // wait 250; copies and data in two separate passes, the keys applied twice,
+  // 275). Batches of 8: 12 and 16 took the same time.
+  static constexpr int kLeafBatch = 8;
   template <int OP>
   MVBT_DEV uint64_t write_chunk(uint32_t key, uint32_t value, uint64_t q, uint32_t leaf,
                                 uint32_t& result, write_ctx& c, const tile_t& t) const {
@@ -1441,13 +1447,11 @@ struct tree_view : tree_ptrs {
   // that owns its group of sorted writes; a split's new right node holds
   // only keys of that group) and no reader runs, while the per-key path and
   // the parents it updates still lock as everywhere else.
-  // The sorted form (PLANNED) takes batches of 8 leaves: its chunks hold few
-  // leaves, and the smaller batch lifts its write pass to 4 waves per SIMD.
   template <int OP, bool PLANNED = false>
   MVBT_DEV uint64_t write_chunk_at(uint32_t key, uint32_t value, uint64_t q, uint32_t leaf, uint32_t cur,
                                    uint32_t& result, write_ctx& c, const tile_t& t,
                                    uint32_t planned = kNone) const {
-    constexpr int LB = PLANNED ? 8 : kLeafBatch;
+    constexpr int LB = kLeafBatch;
     if constexpr (NW > 32) {
       return q;  // 64-pair nodes: register budget; per-key path
     } else {
@@ -1474,46 +1478,38 @@ struct tree_view : tree_ptrs {
       if (locked) stamp_under_lock(c, t);  // one clock read covers every leaf locked above
       if (c.track) cur = c.cur;
       uint64_t pending = locked, prev = 0;
+      uint32_t open = 0;  // leader lane: its leaf's lock word as it is when unlocked
       for (;;) {
-        uint64_t got = 0;
-        {
-          uint64_t m = pending;
-          for (int i = 0; i < LB && m; ++i) {
-            got |= m & (~m + 1);
-            m &= m - 1;
-          }
-        }
-        pending &= ~got;
         // 2. reload this batch's leaves
+        const uint64_t from = pending;
         uint64_t img[LB];
-        uint32_t gl[LB];
-        {
-          uint64_t m = got;
-#pragma unroll
-          for (int i = 0; i < LB; ++i) {
-            gl[i] = m ? (uint32_t)lowest_bit(m) : 0u;
-            if (m) img[i] = ld_coherent(at(t.shfl(leaf, gl[i])) + r);
-            m &= m - 1;
-          }
-        }
-        // 6 (of the previous batch). unlock its leaves once its data stores
-        // are complete: that wait also covers the reloads just issued
-        if (prev) {
-          order_release();
-          if (!PLANNED && ((prev >> r) & 1)) atomic_and32(lock_word(leaf), ~kLockBit);
-        }
-        if (!got) break;
-        const int ng = __builtin_popcountll(got);
-        // 3. plan: apply each leaf's keys in registers; a leaf whose keys do
-        // not all fit (or that no longer covers one of them) goes per key
-        uint32_t ok = 0, changed = 0, need_copy = 0;  // bit i: slot i
 #pragma unroll
         for (int i = 0; i < LB; ++i) {
-          if (i >= ng) continue;
-          node_t n;
-          n.p = img[i];
-          const uint64_t meta = n.meta(t);
-          const uint64_t mem = todo & t.ballot(my_lead == gl[i]);
+          if (pending) img[i] = ld_coherent(at(t.shfl(leaf, (uint32_t)lowest_bit(pending))) + r);
+          pending &= pending - 1;
+        }
+        const uint64_t got = from & ~pending;
+        // 6 (of the previous batch). unlock its leaves once its data stores
+        // are complete: that wait also covers the reloads just issued. A
+        // plain store does it: while the word is locked nobody changes it.
+        order_release();
+        if (!PLANNED && ((prev >> r) & 1)) st32_coherent(lock_word(leaf), open);
+        if (!got) break;
+        // 3. apply each leaf's keys in registers; a leaf whose keys do not all
+        // fit (or that no longer covers one of them) goes per key. 4. The
+        // version copies (new epoch) go out from the images as loaded.
+        uint32_t changed = 0;  // bit i: slot i
+        uint32_t cp = kNone;   // leader lane: copy slot of its leaf
+        uint64_t m = again(got);
+#pragma unroll
+        for (int i = 0; i < LB; ++i, m &= m - 1) {
+          if (!m) continue;
+          const uint32_t l = (uint32_t)lowest_bit(m);
+          node_t o, n;
+          o.p = n.p = img[i];
+          const uint64_t meta = o.meta(t);
+          if (!PLANNED && r == l) open = hi32(meta) & ~kLockBit;
+          const uint64_t mem = todo & t.ballot(my_lead == l);
           bool good = node_t::is_leaf(meta);
           bool chg = false;
           for (uint64_t mm = mem; mm && good; mm &= mm - 1) {
@@ -1535,70 +1531,47 @@ struct tree_view : tree_ptrs {
               chg |= had;
             }
           }
+          if constexpr (VER) {
+            const uint32_t cl = t.shfl(cur, l);
+            if (good && chg && needs_copy_at(o.version(t), cl, t)) {
+              uint32_t slot = PLANNED ? t.shfl(planned, l) : kNone;
+              const bool own = slot == kNone;
+              if (own) slot = alloc(c, t, true);
+              if (slot == kNone) {
+                good = false;  // pool exhausted (flagged): leave the leaf unchanged
+              } else {
+                o.store_unlocked_copy(at(slot), t);
+                if (own) retire(c, slot, t);
+                if (r == l) cp = slot;
+                n.set_lane(node_t::kVerLane, pack(cl, slot), t);
+              }
+            }
+          }
           if (!good) {
             left |= mem;
-          } else {
-            ok |= 1u << i;
-            if (chg) changed |= 1u << i;
-            node_t o;
-            o.p = img[i];
-            if (VER && chg && needs_copy_at(o.version(t), t.shfl(cur, gl[i]), t)) need_copy |= 1u << i;
+          } else if (chg) {
+            changed |= 1u << i;
+            img[i] = n.p;
           }
         }
-        // 4. version copies (new epoch), then their version words
-        uint32_t cp = kNone;  // leader lane: copy slot of its leaf
+        // then their version words
         if constexpr (VER) {
-#pragma unroll
-          for (int i = 0; i < LB; ++i) {
-            if (!((need_copy >> i) & 1)) continue;
-            uint32_t slot = PLANNED ? t.shfl(planned, gl[i]) : kNone;
-            const bool own = slot == kNone;
-            if (own) slot = alloc(c, t, true);
-            if (slot == kNone) {  // pool exhausted (flagged): leave the leaf unchanged
-              ok &= ~(1u << i);
-              changed &= ~(1u << i);
-              need_copy &= ~(1u << i);
-              continue;
-            }
-            node_t n;
-            n.p = img[i];
-            n.store_unlocked_copy(at(slot), t);
-            if (own) retire(c, slot, t);
-            if (r == gl[i]) cp = slot;
-          }
-          if (need_copy) {
+          if (t.any(cp != kNone)) {
             order_release();
             if (cp != kNone) st_coherent(at(leaf) + node_t::kVerLane, pack(cur, cp));
             order_release();
           }
         }
-        // 5. data lanes (the plan re-applied to the loaded image)
+        // 5. data lanes: the whole node goes out as full lines, the metadata
+        // lane as loaded under the lock (unchanged while it is held) and the
+        // version word as just published
+        // (hidden from the compiler: it would keep every leaf's address from
+        // the reload on, two registers each)
+        m = again(got);
+        const uint32_t to = again(leaf);
 #pragma unroll
-        for (int i = 0; i < LB; ++i) {
-          if (!((changed >> i) & 1)) continue;
-          node_t n;
-          n.p = img[i];
-          const uint64_t mem = todo & t.ballot(my_lead == gl[i]);
-          for (uint64_t mm = mem; mm; mm &= mm - 1) {
-            const uint32_t j = (uint32_t)lowest_bit(mm);
-            if (OP == 0) n.insert(t.shfl(key, j), t.shfl(value, j), t);
-            else n.erase(t.shfl(key, j), t);
-          }
-          // The whole node goes out as one full 128-byte line: the metadata
-          // lane as loaded under the lock (unchanged while it is held) and
-          // the version word as just published.
-          // (the shuffles must run on every lane of the tile: a permute reads
-          // nothing from a disabled source lane, and the leader may be one)
-          const uint32_t target = t.shfl(leaf, gl[i]);
-          if constexpr (VER) {
-            const uint32_t cpi = t.shfl(cp, gl[i]), curi = t.shfl(cur, gl[i]);
-            if (((need_copy >> i) & 1) && r == node_t::kVerLane) n.p = pack(curi, cpi);
-          }
-          st_coherent(at(target) + r, n.p);
-        }
-        // keys of leaves that failed for lack of memory go per key (they fail there too)
-        for (int i = 0; i < ng; ++i)
-          if (!((ok >> i) & 1)) left |= todo & t.ballot(my_lead == gl[i]);
+        for (int i = 0; i < LB; ++i, m &= m - 1)
+          if ((changed >> i) & 1) st_coherent(at(t.shfl(to, (uint32_t)lowest_bit(m))) + r, img[i]);
         prev = got;
       }
       return left;

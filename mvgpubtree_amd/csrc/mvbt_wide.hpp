@@ -53,8 +53,8 @@ struct wnode {
   }
   MVBT_DEV static bool data_pair(uint32_t g) { return g < kData; }
   // metadata: pair NW - 1 (last lane, last slot); version word: pair NW - 2
-  MVBT_DEV uint64_t meta(const tile_t& t) const { return t.shfl64(q[P - 1], T - 1); }
-  MVBT_DEV uint64_t version(const tile_t& t) const { return t.shfl64(q[kVerPair % P], kVerPair / P); }
+  MVBT_DEV uint64_t meta(const tile_t& t) const { return t.template bcast64<T - 1>(q[P - 1]); }
+  MVBT_DEV uint64_t version(const tile_t& t) const { return t.template bcast64<kVerPair / P>(q[kVerPair % P]); }
 
   // Child for `key`: value of the last data pair whose pivot <= key (pair 0
   // when none), as node::child_for.
