@@ -874,17 +874,13 @@ __global__ void batch_window_begin_kernel(batch_job* job, uint32_t k) {
 // window's first batch is done, so - when the call may reclaim (no snapshot
 // outside it is live) - every retired copy is garbage: the window's own copies
 // hold contents that only those reads could see. Frees them (appending an
-// epoch to the memory timeline) and merges parked slots either way; the
-// grid part is reclaim_copy_kernel.
-__global__ void batch_window_end_kernel(batch_job* job, tree_state* st, epoch_stat* series) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (ld32_coherent(&job->bad)) {
-    st->scratch[1] = 0;  // reclaim_copy_kernel then copies nothing
-    st->scratch[3] = 0;
-    return;
-  }
+// epoch to the memory timeline) and merges parked slots either way.
+__global__ void __launch_bounds__(kReclaimBlock)
+    batch_window_end_kernel(batch_job* job, tree_state* st, epoch_stat* series, const uint32_t* ring,
+                            const uint32_t* spill, uint32_t* free_stack) {
+  if (ld32_coherent(&job->bad)) return;
   const bool r = job->reclaim != 0;
-  reclaim_prep(st, r ? ~0ull : 0ull, r ? series : nullptr);
+  reclaim_grid(st, r ? ~0ull : 0ull, r ? series : nullptr, ring, spill, free_stack);
 }
 
 // How the sorted form's kernels divide n operations, a count only the device

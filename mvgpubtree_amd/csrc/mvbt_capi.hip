@@ -410,17 +410,14 @@ const dispatch_table* table_for(uint32_t nw, bool versioned) {
 
 bool is_pow2(uint64_t x) { return x && !(x & (x - 1)); }
 
-// Launches the two reclamation kernels: frees ring entries [head, end_pos)
+// Launches the reclamation kernel: frees ring entries [head, end_pos)
 // (end_pos = 0 frees none) and returns parked spill slots to the free stack.
 // A reclamation (record) also appends an epoch to the memory timeline; a
 // spill merge alone does not.
 mvbt_status launch_maintenance(mvbt_tree* t, hipStream_t s, unsigned long long end_pos,
                                const unsigned long long* end_from = nullptr, bool record = false) {
-  hipLaunchKernelGGL(reclaim_prep_kernel, dim3(1), dim3(64), 0, s, t->st, end_pos, end_from,
-                     record ? t->series : nullptr);
-  MVBT_HIP(hipGetLastError());
-  hipLaunchKernelGGL(reclaim_copy_kernel, dim3(t->num_cus * 4), dim3(kBlock), 0, s, t->st,
-                     t->retire_ring, t->spill, t->free_stack);
+  hipLaunchKernelGGL(reclaim_kernel, dim3(kReclaimBlocks), dim3(kReclaimBlock), 0, s, t->st, end_pos, end_from,
+                     record ? t->series : nullptr, t->retire_ring, t->spill, t->free_stack);
   MVBT_HIP(hipGetLastError());
   if (!t->maint_ev) MVBT_HIP(hipEventCreateWithFlags(&t->maint_ev, hipEventDisableTiming));
   MVBT_HIP(hipEventRecord(t->maint_ev, s));
@@ -877,13 +874,11 @@ mvbt_status sorted_tail(mvbt_tree* t, Add& add, batch_job* job, uint32_t which) 
   {
     tree_state* st = t->st;
     epoch_stat* series = t->series;
-    void* eargs[] = {&job, &st, &series};
-    if (hipError_t e = add(reinterpret_cast<void*>(&batch_window_end_kernel), 1, 64, eargs)) return hip_fail(e);
     uint32_t* ring = t->retire_ring;
     uint32_t* spill = t->spill;
     uint32_t* fs = t->free_stack;
-    void* cargs[] = {&st, &ring, &spill, &fs};
-    if (hipError_t e = add(reinterpret_cast<void*>(&reclaim_copy_kernel), (uint32_t)t->num_cus * 4, kBlock, cargs))
+    void* args[] = {&job, &st, &series, &ring, &spill, &fs};
+    if (hipError_t e = add(reinterpret_cast<void*>(&batch_window_end_kernel), kReclaimBlocks, kReclaimBlock, args))
       return hip_fail(e);
   }
   return MVBT_OK;

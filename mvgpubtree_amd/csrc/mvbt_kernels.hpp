@@ -599,7 +599,7 @@ __global__ void __launch_bounds__(256, (kMixedOccupancy<NW, VER, IR>))
 // take_snapshot_kernel (btree_kernels.hpp:473-478): one lane reads the retire
 // ring position, then advances the clock. Synchronous form: both go to the
 // host record `rec`. Stream-ordered form (rec null): the ring position goes
-// to the device slot `pos_slot`, read later by reclaim_prep_kernel, and the
+// to the device slot `pos_slot`, read later by reclaim_kernel, and the
 // id the host already returned (`expected`) is checked against the clock.
 __global__ void snapshot_kernel(tree_state* st, snapshot_record* rec, unsigned long long* pos_slot,
                                 uint32_t expected) {
@@ -617,55 +617,90 @@ __global__ void snapshot_kernel(tree_state* st, snapshot_record* rec, unsigned l
   }
 }
 
-// Reclamation, phase 1 (one lane): frees retire-ring entries [head, end) by
-// moving them onto the free stack. Records the live count before freeing as a
-// peak candidate and, with `series`, appends the epoch to the memory timeline.
-MVBT_DEV void reclaim_prep(tree_state* st, unsigned long long end_pos, epoch_stat* series) {
-  unsigned long long head = st->retire_head, tail = st->retire_tail;
-  unsigned long long end = end_pos < tail ? end_pos : tail;
-  if (end < head) end = head;
-  unsigned long long count = end - head;
+// Reclamation: frees retire-ring entries [head, end) and merges the parked spill
+// slots by moving them onto the free stack; with `series` it appends the epoch
+// to the memory timeline. One launch: every workgroup reads the counters and
+// moves its share, and the last to finish, when all have read them, updates the
+// counters and records the live count before freeing as a peak candidate. (One
+// lane for the counters and a second launch for the entries took 4.2 us for 1000
+// copies and 8.3 for 500K on MI355X, this takes 3.9 and 7.0, one launch and one
+// gap less: a served request of 1000 operations 48 -> 45 us.)
+// Few large workgroups, as each counts itself on one word, about 12 ns apart
+// (500K entries: 1024 workgroups 16 us, 256 8.3, 16 of 1024 threads 15), and
+// eight entries of a thread in flight (one at a time: 10 us).
+constexpr uint32_t kReclaimBlocks = 64, kReclaimBlock = 1024;
+struct reclaim_plan {
+  unsigned long long head, end, count, base, spilled;
+};
+MVBT_DEV reclaim_plan plan_reclaim(const tree_state* st, unsigned long long end_pos) {
+  reclaim_plan p;
+  const unsigned long long tail = st->retire_tail;
+  p.head = st->retire_head;
+  p.end = end_pos < tail ? end_pos : tail;
+  if (p.end < p.head) p.end = p.head;
+  p.count = p.end - p.head;
   // The ring holds at least as many entries as the pool has nodes, so it
   // cannot fill; were it ever to, the positions past head + cap were never
   // stored and their slots still name nodes already freed: free nothing
   // from the ring then (those copies leak instead of being freed twice).
-  if (count > st->retire_cap || (st->error_flags & kErrRetireOverflow)) count = 0;
-  long long top = st->free_top;
-  unsigned long long base = top > 0 ? (unsigned long long)top : 0ull;
-  unsigned long long spilled = st->spill_count;
-  unsigned long long used = st->bump < st->capacity ? st->bump : st->capacity;
-  unsigned long long live = used - base - spilled;
+  if (p.count > st->retire_cap || (st->error_flags & kErrRetireOverflow)) p.count = 0;
+  p.base = st->free_top > 0 ? (unsigned long long)st->free_top : 0ull;
+  p.spilled = st->spill_count;
+  return p;
+}
+MVBT_DEV void commit_reclaim(tree_state* st, const reclaim_plan& p, epoch_stat* series) {
+  const unsigned long long used = st->bump < st->capacity ? st->bump : st->capacity;
+  const unsigned long long live = used - p.base - p.spilled;
   if (live > st->peak_live) st->peak_live = live;
-  st->free_top = (long long)(base + count + spilled);
+  st->free_top = (long long)(p.base + p.count + p.spilled);
   st->spill_count = 0;
   st->settled = used;
-  st->scratch[0] = head;  // first ring position to copy
-  st->scratch[1] = count;
-  st->scratch[2] = base;
-  st->scratch[3] = spilled;
-  st->retire_head = end;
-  st->reclaimed += count;
+  st->retire_head = p.end;
+  st->reclaimed += p.count;
   if (series) {
     const unsigned long long e = st->series_count;
     epoch_stat& x = series[e % kSeriesCap];
     x.epoch = e;
     x.clock = st->clock;
-    x.live_nodes = live - count;
-    x.allocated_total = live - count + st->reclaimed;
-    x.freed_nodes = count;
-    x.retired_pending = tail - end;
+    x.live_nodes = live - p.count;
+    x.allocated_total = live - p.count + st->reclaimed;
+    x.freed_nodes = p.count;
+    x.retired_pending = st->retire_tail - p.end;
     x.reclaimed_total = st->reclaimed;
     x.capacity_nodes = st->capacity;
     st->series_count = e + 1;
   }
 }
+MVBT_DEV void reclaim_grid(tree_state* st, unsigned long long end_pos, epoch_stat* series, const uint32_t* ring,
+                           const uint32_t* spill, uint32_t* free_stack) {
+  const reclaim_plan p = plan_reclaim(st, end_pos);
+  const unsigned long long mask = st->retire_cap - 1;
+  const unsigned long long n = p.count + p.spilled, stride = (unsigned long long)gridDim.x * blockDim.x;
+  constexpr int kEach = 8;  // entries of a thread in flight
+  for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x; i < n; i += kEach * stride) {
+    uint32_t e[kEach];
+#pragma unroll
+    for (int j = 0; j < kEach; ++j) {
+      const unsigned long long x = i + j * stride;
+      if (x < n) e[j] = x < p.count ? ring[(p.head + x) & mask] : spill[x - p.count];
+    }
+#pragma unroll
+    for (int j = 0; j < kEach; ++j)
+      if (i + j * stride < n) free_stack[p.base + i + j * stride] = e[j];
+  }
+  __syncthreads();  // the whole workgroup has read the counters
+  if (threadIdx.x == 0 && atomic_add32(&st->reclaimers, 1u) == gridDim.x - 1) {
+    st->reclaimers = 0;
+    commit_reclaim(st, p, series);
+  }
+}
 
-__global__ void reclaim_prep_kernel(tree_state* st, unsigned long long end_pos, const unsigned long long* end_from,
-                                    epoch_stat* series) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__global__ void __launch_bounds__(kReclaimBlock)
+    reclaim_kernel(tree_state* st, unsigned long long end_pos, const unsigned long long* end_from, epoch_stat* series,
+                   const uint32_t* ring, const uint32_t* spill, uint32_t* free_stack) {
   // the edge recorded on the device by a stream-ordered snapshot
   if (end_from) end_pos = __hip_atomic_load(end_from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  reclaim_prep(st, end_pos, series);
+  reclaim_grid(st, end_pos, series, ring, spill, free_stack);
 }
 
 // Stream-ordered memory statistics (same fields as mvbt_memstats).
@@ -684,19 +719,6 @@ __global__ void stats_kernel(const tree_state* st, unsigned long long node_bytes
   out[5] = st->retire_tail - st->retire_head;
   out[6] = st->reclaimed;
   out[7] = st->retire_tail;
-}
-
-// Reclamation, phase 2: grid-stride copy of the freed ring entries and the
-// parked spill slots onto the free stack.
-__global__ void reclaim_copy_kernel(tree_state* st, const uint32_t* ring, const uint32_t* spill,
-                                    uint32_t* free_stack) {
-  const unsigned long long start = st->scratch[0], count = st->scratch[1], base = st->scratch[2],
-                           spilled = st->scratch[3];
-  const unsigned long long mask = st->retire_cap - 1;
-  for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x;
-       i < count + spilled; i += (unsigned long long)gridDim.x * blockDim.x) {
-    free_stack[base + i] = i < count ? ring[(start + i) & mask] : spill[i - count];
-  }
 }
 
 }  // namespace mvbt
