@@ -8,12 +8,12 @@
 //
 // The layout in memory is the one of mvbt_node.hpp; pair g of a node sits in
 // lane g / P, slot g % P (P = 1, one pair per lane, serves the mixed calls'
-// reader at 16-pair nodes). Two users: reads of launches in which no writer
-// runs (snapshot reads of the versioned tree, plain-tree reads without
-// MVBT_CONCURRENT), through the pass-based reader below, which follows
-// tree_view::read_chunk step for step; and the routing of writers
-// (descend_chunk_wide, coherent loads), whose hints are checked under the
-// leaf lock like those of tree_view::descend_chunk.
+// reader at 16-pair nodes). Users: the pass-based reader below, which follows
+// tree_view::read_chunk step for step, for 32-lane tiles in launches in which no
+// writer runs (16-lane tiles go through mvbt_reads.hpp); the mixed calls'
+// snapshot reads beside writers (read_chunk_wide_conc); and the routing of
+// writers (descend_chunk_wide, coherent loads), whose hints are checked under
+// the leaf lock like those of tree_view::descend_chunk.
 #pragma once
 #include "mvbt_tree.hpp"
 
