@@ -195,13 +195,14 @@ constexpr int range_waves(uint32_t width, bool conc) { return width == 16 && !co
 
 // The same for write and mixed launches: a power of two (so a chunk lies in
 // one aligned group of `width` operations, see superseded()), for 12 waves on
-// each CU while a tile takes one or two and the 16 the kernels hold from there
-// up: with few operations a tile, more tiles cost more on the words they all
-// update than they save (16K updates: 43.6 us at 2 to a tile, 36.8 at 4).
-work_split split_writes(const mvbt_tree* t, uint64_t n, uint32_t width) {
+// each CU while a tile takes one or two and the `waves` the kernel holds from
+// there up: with few operations a tile, more tiles cost more on the words they
+// all update than they save (16K updates: 43.6 us at 2 to a tile, 36.8 at 4).
+// 150K updates of 16-pair leaves: 99 us divided for 16 waves, 80 for 20.
+work_split split_writes(const mvbt_tree* t, uint64_t n, uint32_t width, int waves) {
   work_split ws;
   ws.per_tile = 1;
-  while (ws.per_tile < width && n > (uint64_t)ws.per_tile * t->num_cus * (ws.per_tile < 4 ? 12 : 16) * (64 / width))
+  while (ws.per_tile < width && n > (uint64_t)ws.per_tile * t->num_cus * (ws.per_tile < 4 ? 12 : waves) * (64 / width))
     ws.per_tile *= 2;
   ws.cached = ws.per_tile >= kCachedFrom ? 1u : 0u;
   return ws;
@@ -282,7 +283,7 @@ struct impl {
   template <int OP>
   static mvbt_status write(mvbt_tree* t, const uint32_t* keys, const uint32_t* vals, uint64_t n,
                            hipStream_t s) {
-    const work_split ws = split_writes(t, n, NW);
+    const work_split ws = split_writes(t, n, NW, (kWriteOccupancy<NW, VER>) == 5 ? 20 : 16);
     const uint32_t g = grid_for(t, n, NW, ws.per_tile, 32);
     hipLaunchKernelGGL((write_kernel<NW, VER, OP>), dim3(g), dim3(kBlock), 0, s,
                        t->template view<NW, VER>(), keys, vals, n, ws);
@@ -318,7 +319,7 @@ struct impl {
                            const uint32_t* rhi, uint64_t nr, uint32_t* fout, uint64_t* pairs, uint32_t* counts,
                            uint32_t L, hipStream_t s) {
     if (VER) hipLaunchKernelGGL(mixed_setup_kernel, dim3(1), dim3(64), 0, s, t->st);
-    const work_split ws = split_writes(t, nw + nr, NW);
+    const work_split ws = split_writes(t, nw + nr, NW, 16);
     const uint32_t g = grid_for(t, nw + nr, NW, ws.per_tile, 32);
     hipLaunchKernelGGL((mixed_kernel<NW, VER, IR>), dim3(g), dim3(kBlock), 0, s, t->template view<NW, VER>(), wk, wv,
                        nw, rlo, rhi, nr, fout, pairs, counts, L, ws);

@@ -399,11 +399,15 @@ MVBT_DEV uint32_t write_division(const tree_view<NW, VER>& tv, const work_split&
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)per);  // the same on every lane: kept in a scalar register
 }
 
-// Waves per SIMD the write kernels are held to: plain trees' 16-pair launch
-// needs 96 registers for five (99 cost it 5%: 500K inserts 157 -> 165 us),
-// and so does the mixed insert + range launch at 64 pairs (100 without).
+// Waves per SIMD the write kernels are held to: five (96 registers) at 16-pair
+// nodes (without, versioned ones take 98 to 102: 300K updates 153 us against
+// 131) and at plain 32-pair ones (97: 300K 139 against 122), where launches are
+// then also divided for 20 waves of a CU (split_writes). Versioned 32-pair
+// nodes keep their 104 registers: at five waves two spill, and 300K updates gain
+// (178 -> 160) what 200K to 260K lose (138 -> 142). The mixed insert + range
+// launch at 64 pairs takes 99 without.
 template <int NW, bool VER>
-constexpr int kWriteOccupancy = NW == 16 && !VER ? 5 : 1;
+constexpr int kWriteOccupancy = NW == 16 || (NW == 32 && !VER) ? 5 : 1;
 template <int NW, bool VER, bool IR>
 constexpr int kMixedOccupancy = NW == 64 && VER && IR ? 5 : 1;
 
