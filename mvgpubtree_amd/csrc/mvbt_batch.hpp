@@ -1086,18 +1086,23 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_begin_kernel(batch_jo
   __shared__ uint32_t table[2 * kSmallOps];
   __shared__ uint32_t off[kSmallBatches + 1];
   __shared__ uint32_t wsum[kOpClasses][kWaves];
-  __shared__ uint32_t bad;
+  // Two words: every wave reads the first one below, while others that are ahead
+  // of it may already set the second.
+  __shared__ uint32_t bad_offsets, bad;
   const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6, nb = p.nb, n = (uint32_t)p.nops;
   const unsigned long long first = p.offsets[0];
-  if (tid == 0) bad = p.offsets[nb] - first == p.nops ? 0u : 1u;  // (last < first differs as well)
+  if (tid == 0) {
+    bad_offsets = p.offsets[nb] - first == p.nops ? 0u : 1u;  // (last < first differs as well)
+    bad = 0;
+  }
   __syncthreads();
   for (uint32_t b = tid; b <= nb; b += kSmallBlock) {
     const unsigned long long o = p.offsets[b] - first;
-    if (o > n || (b > 0 && p.offsets[b] < p.offsets[b - 1])) bad = 1;
+    if (o > n || (b > 0 && p.offsets[b] < p.offsets[b - 1])) bad_offsets = 1;
     off[b] = (uint32_t)o;
   }
   __syncthreads();
-  const bool ordered = bad == 0;
+  const bool ordered = bad_offsets == 0;
   uint32_t run[kOpClasses] = {0, 0, 0};
   const op_record* ops = p.ops + first;
   const uint64_t below = (1ull << lane) - 1;
@@ -1188,7 +1193,7 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_begin_kernel(batch_jo
     job->clock0 = clock0;
     job->first_op = first;
     job->nops = ordered ? first + n : first;
-    job->bad = bad;
+    job->bad = bad | bad_offsets;
     job->windows = 1;
     job->reclaim = p.reclaim;
     for (uint32_t q = 0; q < kOpClasses; ++q) {
@@ -1198,7 +1203,7 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_begin_kernel(batch_jo
     job->n_writes = run[0];
     job->n_finds = nf;
     job->n_ranges = nr;
-    if (bad) atomic_or32(&st->error_flags, kErrBadBatch);
+    if (bad | bad_offsets) atomic_or32(&st->error_flags, kErrBadBatch);
   }
 }
 
