@@ -1140,12 +1140,13 @@ constexpr uint64_t kSortedFirstInsert = 64;
 uint32_t default_fill(uint32_t data_lanes) { return (2 * data_lanes + 2) / 3; }
 
 // The sorted form of a tree's first insert. *done: whether it ran; it does not
-// where the pool has no room for the sort behind the nodes, and under stream
-// capture (a replay would load the tree anew over what was written since).
+// where the pool has no room for the sort behind the nodes, from kSortMax keys
+// on, and under stream capture (a replay would load the tree anew over what was
+// written since).
 mvbt_status first_insert(mvbt_tree* t, const uint32_t* keys, const uint32_t* values, uint64_t n, hipStream_t s,
                          bool* done) {
   *done = false;
-  if (n < kSortedFirstInsert || n >= (1ull << 32) - 1) return MVBT_OK;
+  if (n < kSortedFirstInsert || n >= kSortMax) return MVBT_OK;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
     (void)hipGetLastError();

@@ -24,8 +24,11 @@ constexpr uint32_t kSortSegments = 512;  // workgroups (segments) per pass
 constexpr uint32_t kSortBlock = 256;     // threads per workgroup
 constexpr uint32_t kRadix = 256;         // 8-bit digits
 constexpr uint32_t kSortEach = 8;        // elements of a thread in flight
+// Sorts take fewer elements than this: the division below and the indices of the
+// passes' loops, which run up to a chunk past a segment's end, are 32-bit.
+constexpr uint64_t kSortMax = 1ull << 31;
 
-MVBT_DEV void segment_of(uint32_t n, uint32_t g, uint32_t G, uint32_t& a, uint32_t& b) {
+MVBT_HD void segment_of(uint32_t n, uint32_t g, uint32_t G, uint32_t& a, uint32_t& b) {
   const uint32_t seg = (n + G - 1) / G;
   const uint64_t lo = (uint64_t)g * seg;
   a = lo < n ? (uint32_t)lo : n;
