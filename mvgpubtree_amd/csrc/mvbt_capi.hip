@@ -82,10 +82,13 @@ struct mvbt_tree {
   hipStream_t clock_ev_stream = nullptr;
   bool clock_ev_set = false;
   // Free-list maintenance (spill merge, reclamation) must not overlap a
-  // writer on another stream: writers wait for the last maintenance event,
-  // and maintenance runs only when every other stream's last write is done.
+  // writer on another stream, nor another maintenance (its workgroups count
+  // themselves on one word): writers and maintenance wait for the last
+  // maintenance event, and maintenance runs only when every other stream's last
+  // write is done.
   std::map<hipStream_t, hipEvent_t> write_ev;
   hipEvent_t maint_ev = nullptr;
+  hipStream_t maint_stream = nullptr;
   bool spill_maybe = false;
   // Launches with launch-fixed write stamps (batched form, mixed calls) run
   // alone among this handle's writers: they wait for every other stream's
@@ -417,11 +420,18 @@ bool is_pow2(uint64_t x) { return x && !(x & (x - 1)); }
 // spill merge alone does not.
 mvbt_status launch_maintenance(mvbt_tree* t, hipStream_t s, unsigned long long end_pos,
                                const unsigned long long* end_from = nullptr, bool record = false) {
+  if (t->maint_ev && t->maint_stream != s) {
+    // (under capture nothing runs now: a replay is ordered by whoever launches it)
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+    if (cap == hipStreamCaptureStatusNone) MVBT_HIP(hipStreamWaitEvent(s, t->maint_ev, 0));
+  }
   hipLaunchKernelGGL(reclaim_kernel, dim3(kReclaimBlocks), dim3(kReclaimBlock), 0, s, t->st, end_pos, end_from,
                      record ? t->series : nullptr, t->retire_ring, t->spill, t->free_stack);
   MVBT_HIP(hipGetLastError());
   if (!t->maint_ev) MVBT_HIP(hipEventCreateWithFlags(&t->maint_ev, hipEventDisableTiming));
   MVBT_HIP(hipEventRecord(t->maint_ev, s));
+  t->maint_stream = s;
   t->spill_maybe = false;
   return MVBT_OK;
 }

@@ -62,7 +62,7 @@ struct alignas(128) tree_state {
   unsigned long long peak_live;    // max live nodes observed at reclaim/stats
   unsigned long long scratch[4];   // host<->device hand-off words
   uint32_t call_snapshot;          // snapshot reserved by the current mixed call
-  uint32_t reclaimers;             // workgroups done of the running reclamation (0 between launches)
+  uint32_t reclaimers;             // workgroups done of the running reclamation (0 between launches, which never overlap)
   unsigned long long series_count;  // reclamation epochs recorded in the memory timeline
   unsigned long long settled;       // `bump` at the last free-list maintenance, which no write launch overlaps
 };
