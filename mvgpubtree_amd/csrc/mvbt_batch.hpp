@@ -95,7 +95,7 @@ struct alignas(128) batch_job {
   uint32_t n_writes;     // of the current window
   uint32_t n_finds;
   uint32_t n_ranges;
-  uint32_t n_epochs;     // (leaf, batch) groups of the sorted writes: one planned copy slot each
+  uint32_t n_planned;    // small calls: (leaf, batch) groups of the sorted writes with a planned copy slot in w_par
   uint32_t cp_valid;     // planned slots that exist (the rest: pool exhausted)
   uint32_t cp_got;       // of them, taken from the free stack
   uint32_t total_writes;  // write operations of the call (sizes the conflict table)
@@ -109,7 +109,8 @@ struct alignas(128) batch_job {
   uint32_t reclaim;
   uint32_t first[3];     // the window's first write, find and range in their part of `list`
   uint32_t total[3];     // the call's writes, finds and ranges
-  unsigned long long pad4[5];
+  uint32_t small;        // 1: a small call (below)
+  uint32_t pad4[9];
 };
 constexpr uint32_t kFrontierCopies = 8;
 
@@ -155,6 +156,8 @@ __global__ void batch_setup_kernel(batch_job* job, tree_state* st, batch_params 
   job->n_writes = 0;
   job->n_finds = 0;
   job->n_ranges = 0;
+  job->n_planned = 0;
+  job->small = 0;
   job->windows = p.windows > 0 ? p.windows : 1u;
   job->reclaim = p.reclaim;
   if (p.base_out) *p.base_out = job->clock0;  // clock0 goes back to the caller
@@ -876,11 +879,11 @@ __global__ void batch_window_begin_kernel(batch_job* job, uint32_t k) {
 // hold contents that only those reads could see. Frees them (appending an
 // epoch to the memory timeline) and merges parked slots either way.
 __global__ void __launch_bounds__(kReclaimBlock)
-    batch_window_end_kernel(batch_job* job, tree_state* st, epoch_stat* series, const uint32_t* ring,
+    batch_window_end_kernel(batch_job* job, tree_state* st, epoch_stat* series, uint32_t* ring,
                             const uint32_t* spill, uint32_t* free_stack) {
   if (ld32_coherent(&job->bad)) return;
   const bool r = job->reclaim != 0;
-  reclaim_grid(st, r ? ~0ull : 0ull, r ? series : nullptr, ring, spill, free_stack);
+  reclaim_grid(st, r ? ~0ull : 0ull, r ? series : nullptr, ring, spill, free_stack, {job->w_par, job->n_planned});
 }
 
 // How the sorted form's kernels divide n operations, a count only the device
@@ -989,7 +992,6 @@ __global__ void __launch_bounds__(kSortBlock)
   if (ld32_coherent(&job->bad)) return;
   const uint32_t E = scan_row(job->seg, segments, l);
   if (threadIdx.x != kSortBlock - 1) return;
-  job->n_epochs = E;
   tree_state* st = tp.st;
   long long top = atomic_add_s64(&st->free_top, -(long long)E);
   const uint32_t got = (uint32_t)(top < 0 ? 0 : (top > (long long)E ? (long long)E : top));
@@ -1195,6 +1197,8 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_begin_kernel(batch_jo
     job->nops = ordered ? first + n : first;
     job->bad = bad | bad_offsets;
     job->windows = 1;
+    job->n_planned = 0;
+    job->small = 1;
     job->reclaim = p.reclaim;
     for (uint32_t q = 0; q < kOpClasses; ++q) {
       job->first[q] = 0;
@@ -1209,9 +1213,21 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_begin_kernel(batch_jo
 
 // S2. Sort by leaf, gather and copy planning of a small call's writes, by one
 // workgroup: three 8-bit radix passes (bits covers the pool's indices) with
-// leaf and position in LDS, each wave ranking its own stretch; then what
-// batch_gather_kernel, batch_copy_reserve_kernel and batch_assign_kernel do.
-// The sorted leaf hints end in sort_k[1], as after an odd number of passes.
+// leaf and position in LDS, each wave ranking its own stretch; then the gather
+// and the groups as in batch_gather_kernel. The sorted leaf hints end in
+// sort_k[1], as after an odd number of passes.
+// A small call keeps its copies until mvbt_reclaim (unless it may reclaim), so
+// it must not hold more slots than it makes copies: a group's slot is only lent
+// to it. sort_v[0] holds each write's slot, sort_v[1] its group and w_par each
+// group's slot; the write pass sets kSlotUsed there when a copy lies in it, and
+// the end of the call (settle_planned) retires those slots and gives the others
+// back. Until then the call holds a slot per group, so none is planned where
+// the writes could run short of slots for that: a write may take a copy, a new
+// leaf, a new node on each level above, and its tile as many again before it
+// uses them. The write pass then takes slots only for the copies it makes, a
+// few at a time, as a batch-by-batch call would.
+constexpr unsigned long long kPlanRoom = 16;  // free slots a write of the call, plus kPlanRoomBase
+constexpr unsigned long long kPlanRoomBase = 256;
 __global__ void __launch_bounds__(kSmallBlock) batch_small_plan_kernel(batch_job* job, tree_ptrs tp, uint32_t bits) {
   constexpr uint32_t kWaves = kSmallBlock / 64, kItems = kSmallOps / kSmallBlock;
   __shared__ uint32_t key[kSmallOps];
@@ -1220,8 +1236,8 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_plan_kernel(batch_job
   __shared__ uint32_t cnt[kWaves][kRadix];
   __shared__ uint32_t wsum[kWaves];
   __shared__ long long s_top;
-  __shared__ unsigned long long s_bump, s_ring;
-  __shared__ uint32_t s_got, s_valid;
+  __shared__ unsigned long long s_bump;
+  __shared__ uint32_t s_got, s_planned;
   if (ld32_coherent(&job->bad)) return;
   const uint32_t n = job->n_writes;
   if (n == 0) return;
@@ -1307,36 +1323,35 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_plan_kernel(batch_job
     run += total;
   }
   if (tid == 0) {
-    // all of them, or none where the pool has fewer left: the write pass then
-    // takes slots for the copies it does make, as a batch-by-batch call would
     tree_state* st = tp.st;
     const long long on_stack = (long long)ld_coherent((const uint64_t*)&st->free_top);
-    const unsigned long long used = ld_coherent((const uint64_t*)&st->bump);
-    const unsigned long long left = (used < tp.cap_ ? tp.cap_ - used : 0ull) + (on_stack > 0 ? (unsigned long long)on_stack : 0ull);
-    const uint32_t E = left < run ? 0u : run;
-    job->n_epochs = E;
-    s_got = s_valid = 0;
-    if (E) {
-      const long long top = atomic_add_s64(&st->free_top, -(long long)E);
-      const uint32_t got = (uint32_t)(top < 0 ? 0 : (top > (long long)E ? (long long)E : top));
+    const unsigned long long bump = ld_coherent((const uint64_t*)&st->bump);
+    const unsigned long long left = (bump < tp.cap_ ? tp.cap_ - bump : 0ull) + (on_stack > 0 ? (unsigned long long)on_stack : 0ull);
+    s_got = 0;
+    s_planned = left < kPlanRoom * n + kPlanRoomBase ? 0u : run;
+    if (s_planned) {  // (no other writer runs beside the call: what was left is still there)
+      const long long top = atomic_add_s64(&st->free_top, -(long long)run);
+      const uint32_t got = (uint32_t)(top < 0 ? 0 : (top > (long long)run ? (long long)run : top));
       s_top = top;
       s_got = got;
-      if (got < E) s_bump = atomic_add64(&st->bump, (unsigned long long)(E - got));
-      s_valid = E;  // no other writer runs beside the call: what was left is still there
-      s_ring = atomic_add64(&st->retire_tail, (unsigned long long)E);
+      if (got < run) s_bump = atomic_add64(&st->bump, (unsigned long long)(run - got));
     }
+    job->n_planned = s_planned;
   }
   __syncthreads();
-  const unsigned long long mask = tp.retire_cap - 1;
+  const bool planned = s_planned != 0;
 #pragma unroll
   for (uint32_t j = 0; j < kItems; ++j) {
     const uint32_t i = j * kSmallBlock + tid;
     if (i >= n) continue;
     uint32_t slot = kNone;
-    if (group[j] < s_got) slot = ld32_coherent(tp.free_stack + (s_top - 1 - (long long)group[j]));
-    else if (group[j] < s_valid) slot = (uint32_t)(s_bump + (group[j] - s_got));
+    if (planned) {
+      slot = group[j] < s_got ? ld32_coherent(tp.free_stack + (s_top - 1 - (long long)group[j]))
+                              : (uint32_t)(s_bump + (group[j] - s_got));
+      job->sort_v[1][i] = group[j];
+      if (start[j]) job->w_par[group[j]] = slot;
+    }
     job->sort_v[0][i] = slot;
-    if (start[j] && group[j] < s_valid) tp.retire_ring[(s_ring + group[j]) & mask] = slot;
   }
 }
 
@@ -1354,8 +1369,9 @@ __global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, b
   const uint32_t *pars = job->sort_k[which ^ 1u], *slots = job->sort_v[which ^ 1u];
   uint32_t* results = job->results + job->first_op;
   const uint32_t clock0 = job->clock0;
+  const bool lent = job->n_planned != 0;  // slots of a small call: those a copy takes are marked
   write_ctx ctx = tv.begin_writes(t);
-  ctx.exact = 1;
+  ctx.exact = job->small == 0 || lent;  // a small call without a plan: few slots are left, see above
   ctx.track = 0;  // stamps are fixed per batch: clock0 + b + 1
   for (uint64_t p = c.first; p < n; p += c.stride) {
     uint64_t i = p + r;
@@ -1426,6 +1442,7 @@ __global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, b
         R &= ~S;
       }
       if (act) results[rel] = res;
+      if (lent && planned == kTaken) job->w_par[job->sort_v[which][i]] = slots[i] | kSlotUsed;
       if (last) break;
     }
   }

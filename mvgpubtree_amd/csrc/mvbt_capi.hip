@@ -1841,7 +1841,7 @@ mvbt_status mvbt_bulk_build(mvbt_tree* t, const uint32_t* keys, const uint32_t* 
                                           " nodes, the pool has " + std::to_string(t->cfg.pool_nodes));
   hipStream_t s = (hipStream_t)stream;
   // Validate first, so a rejected input leaves the tree untouched and new.
-  unsigned long long* bad = &t->st->scratch[0];
+  unsigned long long* bad = &t->st->bulk_bad;
   MVBT_HIP(hipMemsetAsync(bad, 0, sizeof(*bad), s));
   const uint64_t blocks = std::min<uint64_t>((n + kBlock - 1) / kBlock, (uint64_t)t->num_cus * 8);
   hipLaunchKernelGGL(bulk_check_kernel, dim3((uint32_t)blocks), dim3(kBlock), 0, s, keys,

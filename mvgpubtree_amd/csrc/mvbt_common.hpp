@@ -34,6 +34,7 @@ namespace mvbt {
 constexpr uint32_t kEmpty = 0xFFFFFFFFu;     // empty key / empty value / miss result
 constexpr uint32_t kLatest = 0xFFFFFFFFu;    // snapshot id meaning "latest version"
 constexpr uint32_t kNone = 0xFFFFFFFFu;      // no older version
+constexpr uint32_t kTaken = 0xFFFFFFFEu;     // a planned copy slot that a copy has taken
 constexpr uint32_t kLockBit = 1u << 31;      // metadata value word: lock
 constexpr uint32_t kLeafBit = 1u << 30;      // metadata value word: leaf
 constexpr uint32_t kAboveLeaves = 1u << 29;  // metadata value word: internal node whose children are leaves

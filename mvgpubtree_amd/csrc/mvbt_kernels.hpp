@@ -634,13 +634,21 @@ __global__ void snapshot_kernel(tree_state* st, snapshot_record* rec, unsigned l
 // eight entries of a thread in flight (one at a time: 10 us).
 constexpr uint32_t kReclaimBlocks = 64, kReclaimBlock = 1024;
 struct reclaim_plan {
-  unsigned long long head, end, count, base, spilled;
+  unsigned long long head, end, tail, count, base, spilled;
+};
+// Version-copy slots that a small batched call planned, one per (leaf, batch)
+// group of its writes (mvbt_batch.hpp): kSlotUsed is set where a copy lies in
+// the slot. Node indices are below 2^29.
+constexpr uint32_t kSlotUsed = 0x80000000u;
+struct planned_slots {
+  const uint32_t* slot;
+  uint32_t n;
 };
 MVBT_DEV reclaim_plan plan_reclaim(const tree_state* st, unsigned long long end_pos) {
   reclaim_plan p;
-  const unsigned long long tail = st->retire_tail;
+  p.tail = st->retire_tail;
   p.head = st->retire_head;
-  p.end = end_pos < tail ? end_pos : tail;
+  p.end = end_pos < p.tail ? end_pos : p.tail;
   if (p.end < p.head) p.end = p.head;
   p.count = p.end - p.head;
   // The ring holds at least as many entries as the pool has nodes, so it
@@ -652,31 +660,74 @@ MVBT_DEV reclaim_plan plan_reclaim(const tree_state* st, unsigned long long end_
   p.spilled = st->spill_count;
   return p;
 }
-MVBT_DEV void commit_reclaim(tree_state* st, const reclaim_plan& p, epoch_stat* series) {
+// plan_used copies lie in planned slots, plan_spare planned slots hold none
+// (those were never live); free_used: the copies were freed with the ring's.
+MVBT_DEV void commit_reclaim(tree_state* st, const reclaim_plan& p, epoch_stat* series, unsigned long long plan_used,
+                             unsigned long long plan_spare, bool free_used) {
   const unsigned long long used = st->bump < st->capacity ? st->bump : st->capacity;
-  const unsigned long long live = used - p.base - p.spilled;
+  const unsigned long long live = used - p.base - p.spilled - plan_spare;
+  const unsigned long long freed = p.count + (free_used ? plan_used : 0ull);
   if (live > st->peak_live) st->peak_live = live;
-  st->free_top = (long long)(p.base + p.count + p.spilled);
+  st->free_top = (long long)(p.base + freed + p.spilled + plan_spare);
   st->spill_count = 0;
   st->settled = used;
-  st->retire_head = p.end;
-  st->reclaimed += p.count;
+  st->retire_head = free_used ? p.end + plan_used : p.end;
+  st->retire_tail = p.tail + plan_used;
+  st->reclaimed += freed;
   if (series) {
     const unsigned long long e = st->series_count;
     epoch_stat& x = series[e % kSeriesCap];
     x.epoch = e;
     x.clock = st->clock;
-    x.live_nodes = live - p.count;
-    x.allocated_total = live - p.count + st->reclaimed;
-    x.freed_nodes = p.count;
-    x.retired_pending = st->retire_tail - p.end;
+    x.live_nodes = live - freed;
+    x.allocated_total = live - freed + st->reclaimed;
+    x.freed_nodes = freed;
+    x.retired_pending = st->retire_tail - st->retire_head;
     x.reclaimed_total = st->reclaimed;
     x.capacity_nodes = st->capacity;
     st->series_count = e + 1;
   }
 }
-MVBT_DEV void reclaim_grid(tree_state* st, unsigned long long end_pos, epoch_stat* series, const uint32_t* ring,
-                           const uint32_t* spill, uint32_t* free_stack) {
+// Workgroup 0 deals with the planned slots as well: copies go to the retire ring
+// (or, freed with everything retired, onto the free stack), the others back onto
+// the free stack. Two counters in LDS number them; their order does not matter.
+MVBT_DEV void settle_planned(tree_state* st, const reclaim_plan& p, const planned_slots& planned, bool free_used,
+                             uint32_t* ring, uint32_t* free_stack) {
+  __shared__ uint32_t used, spare;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const unsigned long long mask = st->retire_cap - 1, top = p.base + p.count + p.spilled;
+  const uint64_t below = (1ull << lane) - 1;
+  if (tid == 0) used = spare = 0;
+  __syncthreads();
+  for (uint32_t i0 = 0; i0 < planned.n; i0 += kReclaimBlock) {
+    const bool act = i0 + tid < planned.n;
+    const uint32_t v = act ? planned.slot[i0 + tid] : 0u;
+    const bool u = act && (v & kSlotUsed) != 0;
+    const uint64_t mu = __builtin_amdgcn_ballot_w64(u), ms = __builtin_amdgcn_ballot_w64(act && !u);
+    uint32_t bu = 0, bs = 0;
+    if (lane == 0) {
+      bu = atomicAdd(&used, (uint32_t)__builtin_popcountll(mu));
+      bs = atomicAdd(&spare, (uint32_t)__builtin_popcountll(ms));
+    }
+    bu = (uint32_t)__builtin_amdgcn_readfirstlane((int)bu) + (uint32_t)__builtin_popcountll(mu & below);
+    bs = (uint32_t)__builtin_amdgcn_readfirstlane((int)bs) + (uint32_t)__builtin_popcountll(ms & below);
+    if (free_used) {
+      if (act) free_stack[top + i0 + tid] = v & ~kSlotUsed;
+    } else if (u) {
+      ring[(p.tail + bu) & mask] = v & ~kSlotUsed;
+    } else if (act) {
+      free_stack[top + bs] = v;
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {  // for the workgroup that commits
+    st_coherent(reinterpret_cast<uint64_t*>(&st->plan_used), used);
+    st_coherent(reinterpret_cast<uint64_t*>(&st->plan_spare), spare);
+    order_release();
+  }
+}
+MVBT_DEV void reclaim_grid(tree_state* st, unsigned long long end_pos, epoch_stat* series, uint32_t* ring,
+                           const uint32_t* spill, uint32_t* free_stack, const planned_slots& planned = {}) {
   const reclaim_plan p = plan_reclaim(st, end_pos);
   const unsigned long long mask = st->retire_cap - 1;
   const unsigned long long n = p.count + p.spilled, stride = (unsigned long long)gridDim.x * blockDim.x;
@@ -692,16 +743,24 @@ MVBT_DEV void reclaim_grid(tree_state* st, unsigned long long end_pos, epoch_sta
     for (int j = 0; j < kEach; ++j)
       if (i + j * stride < n) free_stack[p.base + i + j * stride] = e[j];
   }
+  const bool free_used = end_pos == ~0ull;
+  if (planned.n && blockIdx.x == 0) settle_planned(st, p, planned, free_used, ring, free_stack);
   __syncthreads();  // the whole workgroup has read the counters
   if (threadIdx.x == 0 && atomic_add32(&st->reclaimers, 1u) == gridDim.x - 1) {
     st->reclaimers = 0;
-    commit_reclaim(st, p, series);
+    unsigned long long plan_used = 0, plan_spare = 0;
+    if (planned.n) {
+      fence_acquire();
+      plan_used = ld_coherent(reinterpret_cast<const uint64_t*>(&st->plan_used));
+      plan_spare = ld_coherent(reinterpret_cast<const uint64_t*>(&st->plan_spare));
+    }
+    commit_reclaim(st, p, series, plan_used, plan_spare, free_used);
   }
 }
 
 __global__ void __launch_bounds__(kReclaimBlock)
     reclaim_kernel(tree_state* st, unsigned long long end_pos, const unsigned long long* end_from, epoch_stat* series,
-                   const uint32_t* ring, const uint32_t* spill, uint32_t* free_stack) {
+                   uint32_t* ring, const uint32_t* spill, uint32_t* free_stack) {
   // the edge recorded on the device by a stream-ordered snapshot
   if (end_from) end_pos = __hip_atomic_load(end_from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   reclaim_grid(st, end_pos, series, ring, spill, free_stack);

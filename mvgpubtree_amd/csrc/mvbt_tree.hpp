@@ -60,7 +60,8 @@ struct alignas(128) tree_state {
   unsigned long long retire_cap;   // ring capacity (power of two)
   unsigned long long reclaimed;    // total nodes returned to the free stack
   unsigned long long peak_live;    // max live nodes observed at reclaim/stats
-  unsigned long long scratch[4];   // host<->device hand-off words
+  unsigned long long bulk_bad;     // bulk build: its input is not strictly ascending
+  unsigned long long plan_used, plan_spare;  // of a small batched call's planned copy slots (reclaim_grid)
   uint32_t call_snapshot;          // snapshot reserved by the current mixed call
   uint32_t reclaimers;             // workgroups done of the running reclamation (0 between launches, which never overlap)
   unsigned long long series_count;  // reclamation epochs recorded in the memory timeline
@@ -1433,15 +1434,17 @@ struct tree_view : tree_ptrs {
   template <int OP>
   MVBT_DEV uint64_t write_chunk(uint32_t key, uint32_t value, uint64_t q, uint32_t leaf,
                                 uint32_t& result, write_ctx& c, const tile_t& t) const {
-    return write_chunk_at<OP>(key, value, q, leaf, c.cur, result, c, t);
+    uint32_t none = kNone;
+    return write_chunk_at<OP>(key, value, q, leaf, c.cur, result, c, t, none);
   }
   // The same with a stamp per lane (`cur`, equal for the lanes of one leaf):
   // the sorted batched form writes several batches' epochs in one chunk.
   // A tile that tracks the clock (c.track) uses c.cur for every lane.
   // PLANNED: `planned` (per lane, equal for the lanes of one leaf) is the
-  // version-copy slot reserved for the leaf's epoch ahead of the launch and
-  // already entered in the retire ring, so no copy allocates or retires here
-  // (kNone: none was reserved, and the tile allocates if the leaf needs it).
+  // version-copy slot reserved for the leaf's epoch ahead of the launch, so no
+  // copy allocates or retires here (kNone: none was reserved, and the tile
+  // allocates if the leaf needs it). The leader lane of a leaf whose copy went
+  // there gets kTaken.
   // PLANNED also takes no leaf locks:
   // in the sorted form's write pass every leaf has one writing tile (the one
   // that owns its group of sorted writes; a split's new right node holds
@@ -1449,8 +1452,7 @@ struct tree_view : tree_ptrs {
   // the parents it updates still lock as everywhere else.
   template <int OP, bool PLANNED = false>
   MVBT_DEV uint64_t write_chunk_at(uint32_t key, uint32_t value, uint64_t q, uint32_t leaf, uint32_t cur,
-                                   uint32_t& result, write_ctx& c, const tile_t& t,
-                                   uint32_t planned = kNone) const {
+                                   uint32_t& result, write_ctx& c, const tile_t& t, uint32_t& planned) const {
     constexpr int LB = kLeafBatch;
     if constexpr (NW > 32) {
       return q;  // 64-pair nodes: register budget; per-key path
@@ -1535,13 +1537,14 @@ struct tree_view : tree_ptrs {
             const uint32_t cl = t.shfl(cur, l);
             if (good && chg && needs_copy_at(o.version(t), cl, t)) {
               uint32_t slot = PLANNED ? t.shfl(planned, l) : kNone;
-              const bool own = slot == kNone;
+              const bool own = slot >= kTaken;
               if (own) slot = alloc(c, t, true);
               if (slot == kNone) {
                 good = false;  // pool exhausted (flagged): leave the leaf unchanged
               } else {
                 o.store_unlocked_copy(at(slot), t);
                 if (own) retire(c, slot, t);
+                else if (r == l) planned = kTaken;
                 if (r == l) cp = slot;
                 n.set_lane(node_t::kVerLane, pack(cl, slot), t);
               }

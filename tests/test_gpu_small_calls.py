@@ -57,3 +57,129 @@ def test_unknown_types_reject_a_call_of_many_waves(dev, n, where):
     assert tree.error_flags() == 0
     assert np.array_equal(to_np(res), want)
     assert tree.validate_tree_structure()[0] == ref.size()
+
+
+def _update_ops(rng, init, n, nb, noop):
+    """nb batches of writes: updates and erases of present keys, each batch its
+    own distinct keys, and a share `noop` of erases of absent keys."""
+    ops, offs = [], [0]
+    absent = wl.absent_keys(rng, n, init)
+    at = 0
+    for m in np.diff(np.linspace(0, n, nb + 1).astype(int)):
+        k = int(m * noop)
+        o = np.zeros((m, 4), np.uint32)
+        o[:k, 0], o[:k, 1] = mv.OP_ERASE, absent[at:at + k]
+        o[k:, 0], o[k:, 1] = mv.OP_INSERT, rng.choice(init, size=m - k, replace=False)
+        o[k:, 2] = rng.integers(1, 1 << 31, size=m - k)
+        at += k
+        ops.append(o[rng.permutation(m)])
+        offs.append(offs[-1] + m)
+    return np.concatenate(ops), np.array(offs, np.uint64)
+
+
+@pytest.mark.parametrize("nw", [16, 32, 64])
+@pytest.mark.parametrize("n,nb", [(1, 1), (300, 3), (1025, 1), (9000, 40), (16383, 3)])
+@pytest.mark.parametrize("noop", [0.0, 0.7, 1.0])
+def test_slots_taken_are_the_copies_made(dev, nw, n, nb, noop):
+    """Calls in the default mode retire as many slots as a call that runs
+    batch after batch: one per copy of a leaf, none for writes that change
+    nothing; the others are free again when the call ends, also under a live
+    snapshot, and a reclamation gives the copies' back."""
+    rng = np.random.default_rng(n + nw)
+    init = np.sort(wl.unique_keys(rng, 40_000))
+    ops, offs = _update_ops(rng, init, n, nb, noop)
+    seen = []
+    for mode in (0, 3):
+        tree = mv.GpuVersionedBTree(pool_nodes=1 << 19, node_width=nw)
+        tree.set_worker_mode(mode)
+        tree.bulk_build(to_dev(init, dev), to_dev(wl.value_of(init), dev))
+        live = tree.memory_stats().live_nodes
+        snap = tree.take_snapshot()
+        stats = []
+        for _ in range(3):
+            tree.run_batches(to_dev(ops, dev), to_dev(offs, dev))
+            st = tree.memory_stats()
+            stats.append((st.retired_total, st.live_nodes))
+            assert st.live_nodes + st.free_nodes == st.capacity_nodes
+            assert st.live_nodes == live + st.retired_pending
+        if noop == 1.0:
+            assert stats[-1] == (0, live)
+        assert tree.memory_stats().peak_live_nodes == stats[-1][1]
+        seen.append((stats, tree.export()))
+        tree.release_snapshot(snap)
+        tree.reclaim()
+        st = tree.memory_stats()
+        assert st.live_nodes == live and st.retired_pending == 0 and st.reclaimed_nodes == st.retired_total
+        # the free slots are distinct: every one can be used, and the tree stays whole
+        tree.insert(to_dev(init, dev), to_dev(wl.value_of(init), dev))
+        assert tree.error_flags() == 0
+        assert np.array_equal(to_np(tree.find(to_dev(init, dev))), wl.value_of(init))
+        assert tree.validate_tree_structure()[0] == init.size
+    assert seen[0][0] == seen[1][0]
+    assert np.array_equal(seen[0][1], seen[1][1])
+
+
+@pytest.mark.parametrize("no_alloc", [False, True])
+def test_slots_of_calls_that_reclaim(dev, no_alloc):
+    """Small calls of the sorted form that reclaim in the call free the copies
+    they made, and record the epoch."""
+    rng = np.random.default_rng(3)
+    init = np.sort(wl.unique_keys(rng, 40_000))
+    tree = mv.GpuVersionedBTree(pool_nodes=1 << 17, node_width=32)
+    tree.set_worker_mode(2)
+    tree.bulk_build(to_dev(init, dev), to_dev(wl.value_of(init), dev))
+    live = tree.memory_stats().live_nodes
+    total = 0
+    for k, (n, nb) in enumerate([(900, 3), (16384, 30), (1, 1), (5000, 4096)]):
+        ops, offs = _update_ops(rng, init, n, nb, 0.5)
+        ref = mv.GpuVersionedBTree(pool_nodes=1 << 18, node_width=32)
+        ref.set_worker_mode(0)
+        ref.bulk_build(to_dev(init, dev), to_dev(wl.value_of(init), dev))
+        ref.run_batches(to_dev(ops, dev), to_dev(offs, dev))
+        total += ref.memory_stats().retired_total
+        tree.run_batches(to_dev(ops, dev), to_dev(offs, dev), no_alloc=no_alloc)
+        st = tree.memory_stats()
+        assert st.live_nodes == live and st.retired_pending == 0
+        assert st.live_nodes + st.free_nodes == st.capacity_nodes
+        assert st.retired_total == st.reclaimed_nodes == total
+        assert tree.memory_series()[-1].freed_nodes == ref.memory_stats().retired_total
+    assert tree.error_flags() == 0
+    assert tree.validate_tree_structure()[0] == init.size
+
+
+@pytest.mark.parametrize("fill", [0, 14])
+def test_nearly_full_pools(dev, fill):
+    """A call of erases of absent keys, updates and inserts that split (at
+    fill 14 every node of every level is full) into pools of every spare size:
+    where the form that takes a slot only for what it stores finds room, the
+    default form does."""
+    rng = np.random.default_rng(17)
+    init = np.sort(wl.unique_keys(rng, 20_000))
+    vals = wl.value_of(init)
+    probe = mv.GpuVersionedBTree(pool_nodes=1 << 14)
+    probe.bulk_build(to_dev(init, dev), to_dev(vals, dev), fill=fill)
+    live = probe.memory_stats().live_nodes
+    for n, inserts in ((1, 1), (40, 40), (2000, 60)):
+        absent = wl.absent_keys(rng, n, init)
+        ops = np.zeros((n, 4), np.uint32)
+        ops[:, 0], ops[:, 1] = mv.OP_ERASE, absent
+        ops[:inserts, 0], ops[:inserts, 2] = mv.OP_INSERT, 7
+        ops = ops[rng.permutation(n)]
+        offs = np.array([0, n // 2, n], np.uint64)
+        leaf = np.searchsorted(init[::fill or 10], ops[:, 1], side="right")
+        groups = len(set(zip(leaf.tolist(), (np.arange(n) >= n // 2).tolist())))  # (leaf, batch) pairs written
+        near = [groups + k for k in (-1, 0, 1, 5, 20, 60, 130, 200, 300)]
+        for spare in near + [4, 8, 16, 40, 80, 120, 160, 240, 400, 900, 4200, 6500, 30_000, 33_000]:
+            if spare < 2:
+                continue
+            flags = []
+            for mode in (0, 3):
+                tree = mv.GpuVersionedBTree(pool_nodes=live + spare)
+                tree.set_worker_mode(mode)
+                tree.bulk_build(to_dev(init, dev), to_dev(vals, dev), fill=fill)
+                res = to_np(tree.run_batches(to_dev(ops, dev), to_dev(offs, dev)))
+                flags.append(tree.error_flags())
+                if flags[-1] == 0:
+                    assert np.array_equal(res, (ops[:, 0] == mv.OP_INSERT).astype(np.uint32))
+                    assert tree.validate_tree_structure()[0] == init.size + inserts
+            assert flags[1] == 0 or flags[0] != 0, (n, spare, flags)
