@@ -95,7 +95,7 @@ struct alignas(128) batch_job {
   uint32_t n_writes;     // of the current window
   uint32_t n_finds;
   uint32_t n_ranges;
-  uint32_t n_planned;    // small calls: (leaf, batch) groups of the sorted writes with a planned copy slot in w_par
+  uint32_t n_planned;    // lent slots: (leaf, batch) groups of the window's writes, each one's slot in w_par
   uint32_t cp_valid;     // planned slots that exist (the rest: pool exhausted)
   uint32_t cp_got;       // of them, taken from the free stack
   uint32_t total_writes;  // write operations of the call (sizes the conflict table)
@@ -109,7 +109,7 @@ struct alignas(128) batch_job {
   uint32_t reclaim;
   uint32_t first[3];     // the window's first write, find and range in their part of `list`
   uint32_t total[3];     // the call's writes, finds and ranges
-  uint32_t small;        // 1: a small call (below)
+  uint32_t lend;         // 1: copy slots are lent to the call (lend_slots)
   uint32_t pad4[9];
 };
 constexpr uint32_t kFrontierCopies = 8;
@@ -127,6 +127,7 @@ struct batch_params {
   uint32_t hash_mask;
   uint32_t windows;  // sorted form: windows of batches the call runs in (>= 1)
   uint32_t reclaim;  // sorted form: free every retired copy after each window
+  uint32_t lend;     // sorted form: see lend_slots (small calls: always)
 };
 
 // 1. Parameters in, clock range reserved, queue reset.
@@ -157,7 +158,7 @@ __global__ void batch_setup_kernel(batch_job* job, tree_state* st, batch_params 
   job->n_finds = 0;
   job->n_ranges = 0;
   job->n_planned = 0;
-  job->small = 0;
+  job->lend = p.lend;
   job->windows = p.windows > 0 ? p.windows : 1u;
   job->reclaim = p.reclaim;
   if (p.base_out) *p.base_out = job->clock0;  // clock0 goes back to the caller
@@ -983,15 +984,39 @@ __global__ void __launch_bounds__(kSortBlock) batch_gather_kernel(batch_job* job
   }
 }
 
+// Calls that keep their copies until mvbt_reclaim however small they are (mode 3
+// below 16384 operations), and all small calls, must not hold more slots than
+// they make copies: there a group's slot is only lent to the call. sort_v holds
+// each write's slot in one buffer and its group in the other, w_par each group's
+// slot; the write pass sets kSlotUsed there when a copy lies in it, and the end
+// of the window (settle_planned) retires those slots and gives the others back.
+// Until then the call holds a slot per group, so none is planned where its
+// writes could run short of slots for that: a write may take a copy, a new leaf,
+// a new node on each level above, and its tile as many again before it uses
+// them. The write pass then takes slots only for the copies it makes, a few at a
+// time, as a batch-by-batch call would.
+constexpr unsigned long long kPlanRoom = 16;  // free slots a write of the window, plus kPlanRoomBase
+constexpr unsigned long long kPlanRoomBase = 256;
+MVBT_DEV bool lend_slots(const tree_ptrs& tp, uint32_t writes) {
+  const long long on_stack = (long long)ld_coherent((const uint64_t*)&tp.st->free_top);
+  const unsigned long long bump = ld_coherent((const uint64_t*)&tp.st->bump);
+  const unsigned long long fresh = bump < tp.cap_ ? tp.cap_ - bump : 0ull;
+  return fresh + (on_stack > 0 ? (unsigned long long)on_stack : 0ull) >= kPlanRoom * writes + kPlanRoomBase;
+}
+
 // One workgroup: seg to each segment's first group number; its last thread,
 // which holds the number of groups, reserves a slot for each (free stack first,
-// then the frontier) and as many retire-ring positions as slots exist.
+// then the frontier) and, unless they are lent, as many retire-ring positions as
+// slots exist.
 __global__ void __launch_bounds__(kSortBlock)
     batch_copy_reserve_kernel(batch_job* job, tree_ptrs tp, uint32_t segments) {
   __shared__ scan_lds l;
   if (ld32_coherent(&job->bad)) return;
-  const uint32_t E = scan_row(job->seg, segments, l);
+  const uint32_t groups = scan_row(job->seg, segments, l);
   if (threadIdx.x != kSortBlock - 1) return;
+  const bool lend = job->lend != 0;
+  const uint32_t E = !lend || lend_slots(tp, job->n_writes) ? groups : 0u;
+  job->n_planned = lend ? E : 0u;
   tree_state* st = tp.st;
   long long top = atomic_add_s64(&st->free_top, -(long long)E);
   const uint32_t got = (uint32_t)(top < 0 ? 0 : (top > (long long)E ? (long long)E : top));
@@ -1000,7 +1025,7 @@ __global__ void __launch_bounds__(kSortBlock)
   const unsigned long long fresh = b < (unsigned long long)tp.cap_ ? (unsigned long long)tp.cap_ - b : 0ull;
   const uint32_t valid = got + (uint32_t)((unsigned long long)(E - got) < fresh ? (E - got) : fresh);
   if (valid < E) atomic_or32(&st->error_flags, kErrPoolExhausted);
-  const unsigned long long ring = atomic_add64(&st->retire_tail, (unsigned long long)valid);
+  const unsigned long long ring = lend ? 0ull : atomic_add64(&st->retire_tail, (unsigned long long)valid);
   job->cp_top = top;
   job->cp_got = got;
   job->cp_bump = b;
@@ -1009,7 +1034,8 @@ __global__ void __launch_bounds__(kSortBlock)
 }
 
 // The slot of every sorted write's group (kNone past the pool); the existing
-// ones go to the retire ring, each by its group's first write.
+// ones go to the retire ring (lent ones to w_par), each by its group's first
+// write.
 __global__ void __launch_bounds__(kSortBlock) batch_assign_kernel(batch_job* job, tree_ptrs tp, uint32_t which) {
   constexpr uint32_t kWaves = kSortBlock / 64;
   __shared__ uint32_t wsum[kWaves];
@@ -1018,6 +1044,7 @@ __global__ void __launch_bounds__(kSortBlock) batch_assign_kernel(batch_job* job
   const long long top = job->cp_top;
   const unsigned long long bump = job->cp_bump, ring = job->cp_ring, mask = tp.retire_cap - 1;
   uint32_t* slots = job->sort_v[which ^ 1u];
+  const bool lent = job->n_planned != 0;
   const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const uint64_t below = (1ull << lane) - 1;
   uint32_t a, e;
@@ -1042,7 +1069,12 @@ __global__ void __launch_bounds__(kSortBlock) batch_assign_kernel(batch_job* job
       if (k < got) slot = ld32_coherent(tp.free_stack + (top - 1 - (long long)k));
       else if (k < valid) slot = (uint32_t)(bump + (k - got));
       slots[i] = slot;
-      if (start && k < valid) tp.retire_ring[(ring + k) & mask] = slot;
+      if (lent) {
+        job->sort_v[which][i] = k;
+        if (start) job->w_par[k] = slot;
+      } else if (start && k < valid) {
+        tp.retire_ring[(ring + k) & mask] = slot;
+      }
     }
     run += tot;
     __syncthreads();
@@ -1198,7 +1230,7 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_begin_kernel(batch_jo
     job->bad = bad | bad_offsets;
     job->windows = 1;
     job->n_planned = 0;
-    job->small = 1;
+    job->lend = 1;
     job->reclaim = p.reclaim;
     for (uint32_t q = 0; q < kOpClasses; ++q) {
       job->first[q] = 0;
@@ -1216,18 +1248,6 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_begin_kernel(batch_jo
 // leaf and position in LDS, each wave ranking its own stretch; then the gather
 // and the groups as in batch_gather_kernel. The sorted leaf hints end in
 // sort_k[1], as after an odd number of passes.
-// A small call keeps its copies until mvbt_reclaim (unless it may reclaim), so
-// it must not hold more slots than it makes copies: a group's slot is only lent
-// to it. sort_v[0] holds each write's slot, sort_v[1] its group and w_par each
-// group's slot; the write pass sets kSlotUsed there when a copy lies in it, and
-// the end of the call (settle_planned) retires those slots and gives the others
-// back. Until then the call holds a slot per group, so none is planned where
-// the writes could run short of slots for that: a write may take a copy, a new
-// leaf, a new node on each level above, and its tile as many again before it
-// uses them. The write pass then takes slots only for the copies it makes, a
-// few at a time, as a batch-by-batch call would.
-constexpr unsigned long long kPlanRoom = 16;  // free slots a write of the call, plus kPlanRoomBase
-constexpr unsigned long long kPlanRoomBase = 256;
 __global__ void __launch_bounds__(kSmallBlock) batch_small_plan_kernel(batch_job* job, tree_ptrs tp, uint32_t bits) {
   constexpr uint32_t kWaves = kSmallBlock / 64, kItems = kSmallOps / kSmallBlock;
   __shared__ uint32_t key[kSmallOps];
@@ -1324,11 +1344,8 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_plan_kernel(batch_job
   }
   if (tid == 0) {
     tree_state* st = tp.st;
-    const long long on_stack = (long long)ld_coherent((const uint64_t*)&st->free_top);
-    const unsigned long long bump = ld_coherent((const uint64_t*)&st->bump);
-    const unsigned long long left = (bump < tp.cap_ ? tp.cap_ - bump : 0ull) + (on_stack > 0 ? (unsigned long long)on_stack : 0ull);
     s_got = 0;
-    s_planned = left < kPlanRoom * n + kPlanRoomBase ? 0u : run;
+    s_planned = lend_slots(tp, n) ? run : 0u;
     if (s_planned) {  // (no other writer runs beside the call: what was left is still there)
       const long long top = atomic_add_s64(&st->free_top, -(long long)run);
       const uint32_t got = (uint32_t)(top < 0 ? 0 : (top > (long long)run ? (long long)run : top));
@@ -1369,9 +1386,9 @@ __global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, b
   const uint32_t *pars = job->sort_k[which ^ 1u], *slots = job->sort_v[which ^ 1u];
   uint32_t* results = job->results + job->first_op;
   const uint32_t clock0 = job->clock0;
-  const bool lent = job->n_planned != 0;  // slots of a small call: those a copy takes are marked
+  const bool lent = job->n_planned != 0;  // slots that a copy takes are marked
   write_ctx ctx = tv.begin_writes(t);
-  ctx.exact = job->small == 0 || lent;  // a small call without a plan: few slots are left, see above
+  ctx.exact = job->lend == 0 || lent;  // else few slots are left (lend_slots)
   ctx.track = 0;  // stamps are fixed per batch: clock0 + b + 1
   for (uint64_t p = c.first; p < n; p += c.stride) {
     uint64_t i = p + r;

@@ -1548,7 +1548,8 @@ mvbt_status mvbt_run_batches(mvbt_tree* t, const mvbt_op* ops, uint64_t num_ops,
   p.base_out = snapshot_base;
   p.hash_mask = (uint32_t)(conflict_entries(num_ops) - 1);
   p.windows = windows_for(t, num_ops, num_batches);
-  p.reclaim = may_reclaim_in_call(t, flags) && !keeps_copies(t, num_ops) ? 1u : 0u;
+  p.lend = keeps_copies(t, num_ops) ? 1u : 0u;
+  p.reclaim = may_reclaim_in_call(t, flags) && !p.lend ? 1u : 0u;
   if (flags & MVBT_USE_GRAPH) {
     const uint32_t gi = graph_index(t, p.windows);
     if (!t->graph_exec[gi]) {

@@ -636,8 +636,8 @@ constexpr uint32_t kReclaimBlocks = 64, kReclaimBlock = 1024;
 struct reclaim_plan {
   unsigned long long head, end, tail, count, base, spilled;
 };
-// Version-copy slots that a small batched call planned, one per (leaf, batch)
-// group of its writes (mvbt_batch.hpp): kSlotUsed is set where a copy lies in
+// Version-copy slots lent to a batched call, one per (leaf, batch) group of its
+// writes (lend_slots in mvbt_batch.hpp): kSlotUsed is set where a copy lies in
 // the slot. Node indices are below 2^29.
 constexpr uint32_t kSlotUsed = 0x80000000u;
 struct planned_slots {

@@ -61,7 +61,7 @@ struct alignas(128) tree_state {
   unsigned long long reclaimed;    // total nodes returned to the free stack
   unsigned long long peak_live;    // max live nodes observed at reclaim/stats
   unsigned long long bulk_bad;     // bulk build: its input is not strictly ascending
-  unsigned long long plan_used, plan_spare;  // of a small batched call's planned copy slots (reclaim_grid)
+  unsigned long long plan_used, plan_spare;  // of the slots lent to a batched call (settle_planned)
   uint32_t call_snapshot;          // snapshot reserved by the current mixed call
   uint32_t reclaimers;             // workgroups done of the running reclamation (0 between launches, which never overlap)
   unsigned long long series_count;  // reclamation epochs recorded in the memory timeline

@@ -183,3 +183,37 @@ def test_nearly_full_pools(dev, fill):
                     assert np.array_equal(res, (ops[:, 0] == mv.OP_INSERT).astype(np.uint32))
                     assert tree.validate_tree_structure()[0] == init.size + inserts
             assert flags[1] == 0 or flags[0] != 0, (n, spare, flags)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("spare", [3600, 200_000])
+def test_few_operations_in_many_batches(dev, spare, graph):
+    """Fewer than 16384 operations in more batches than the small form takes:
+    the default mode holds a slot only for a copy it makes there too, so the
+    call fits a pool that has room for its copies and not for its writes, and
+    gives back what it did not use of a larger one; in one window and several."""
+    rng = np.random.default_rng(23)
+    init = np.sort(wl.unique_keys(rng, 20_000))
+    n, nb = 9000, 5000
+    ops, _ = _update_ops(rng, init, n, 1, 0.9)
+    offs = np.concatenate([[0], np.sort(rng.integers(0, n + 1, size=nb - 1)), [n]]).astype(np.uint64)
+    probe = mv.GpuVersionedBTree(pool_nodes=1 << 14)
+    probe.bulk_build(to_dev(init, dev), to_dev(wl.value_of(init), dev))
+    live = probe.memory_stats().live_nodes
+    want, _, ref = oracle.replay_batches(init, wl.value_of(init), ops, offs, 1, 1)
+    tree = mv.GpuVersionedBTree(pool_nodes=live + spare)
+    tree.bulk_build(to_dev(init, dev), to_dev(wl.value_of(init), dev))
+    if graph:
+        tree.reserve_batches(20_000, nb)  # a larger call's reservation covers it
+    tree.set_batch_window(4000 if graph else 0)
+    for k in range(2):  # (the second call finds the present keys updated and the absent ones absent as well)
+        res = to_np(tree.run_batches(to_dev(ops, dev), to_dev(offs, dev), use_graph=graph))
+        assert tree.error_flags() == 0
+        assert np.array_equal(res, want)
+        st = tree.memory_stats()
+        assert 0 < st.retired_total <= (k + 1) * n // 10
+        assert st.live_nodes == live + st.retired_total == st.capacity_nodes - st.free_nodes
+    tree.reclaim()
+    st = tree.memory_stats()
+    assert st.live_nodes == live and st.reclaimed_nodes == st.retired_total
+    assert tree.validate_tree_structure()[0] == ref.size()
