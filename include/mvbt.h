@@ -306,6 +306,10 @@ typedef struct mvbt_op {
  * issued later on other streams (other run_batches calls included) wait for it. User
  * kernels that write through a device view (mvbt_device_view) must not overlap it
  * either (its reads and its sorted-form leaf writes assume no other writer runs).
+ * MVBT_CONCURRENT snapshot reads on other streams may overlap it. Reads of the latest
+ * version may overlap calls of fewer than 16384 operations, which lock the leaves they
+ * write as every other write does, but not larger ones in the sorted form: those write
+ * whole leaves without their locks, and a read that holds one may leave it locked.
  * Versioned trees only; scratch for num_batches and num_ops is allocated on first use
  * and when a call needs more (synchronous then). */
 mvbt_status mvbt_run_batches(mvbt_tree* tree, const mvbt_op* ops, uint64_t num_ops,

@@ -1372,10 +1372,13 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_plan_kernel(batch_job
   }
 }
 
-// 8. The write pass over the sorted writes (buffers sort_k/v[which]).
-template <int NW>
-__global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, batch_job* job, uint32_t which) {
-  if (ld32_coherent(&job->bad)) return;
+// 8. The write pass over the sorted writes (buffers sort_k/v[which]). LEND: slots
+// are lent to the call (lend_slots), and leaves are locked, for latest reads on
+// other streams: such calls once ran on the persistent worker, which locks them.
+// It is 1% of a small call's time and 4.6% of 4M operations' (1273 -> 1332 us),
+// whose leaves were never locked: mvbt_run_batches forbids such reads beside them.
+template <int NW, bool LEND>
+MVBT_DEV void sorted_writes(const tree_ptrs& tp, batch_job* job, uint32_t which) {
   const tree_view<NW, true> tv(tp);
   tile<NW> t;
   const uint32_t r = t.rank();
@@ -1386,9 +1389,9 @@ __global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, b
   const uint32_t *pars = job->sort_k[which ^ 1u], *slots = job->sort_v[which ^ 1u];
   uint32_t* results = job->results + job->first_op;
   const uint32_t clock0 = job->clock0;
-  const bool lent = job->n_planned != 0;  // slots that a copy takes are marked
+  const bool lent = LEND && job->n_planned != 0;  // slots that a copy takes are marked
   write_ctx ctx = tv.begin_writes(t);
-  ctx.exact = job->lend == 0 || lent;  // else few slots are left (lend_slots)
+  ctx.exact = !LEND || lent;  // else few slots are left
   ctx.track = 0;  // stamps are fixed per batch: clock0 + b + 1
   for (uint64_t p = c.first; p < n; p += c.stride) {
     uint64_t i = p + r;
@@ -1443,8 +1446,8 @@ __global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, b
           uint64_t q = t.ballot(sel && op.type == (w == 0 ? kOpInsert : kOpErase));
           if (!q) continue;
           ctx.want = (uint32_t)__builtin_popcountll(q);
-          q = (w == 0) ? tv.template write_chunk_at<0, true>(op.key, op.arg, q, leaf, cur, res, ctx, t, planned)
-                       : tv.template write_chunk_at<1, true>(op.key, 0u, q, leaf, cur, res, ctx, t, planned);
+          q = (w == 0) ? tv.template write_chunk_at<0, true, LEND>(op.key, op.arg, q, leaf, cur, res, ctx, t, planned)
+                       : tv.template write_chunk_at<1, true, LEND>(op.key, 0u, q, leaf, cur, res, ctx, t, planned);
           while (q) {
             const uint32_t j = (uint32_t)lowest_bit(q);
             ctx.want = (uint32_t)__builtin_popcountll(q);
@@ -1464,6 +1467,12 @@ __global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, b
     }
   }
   tv.finish(ctx, t);
+}
+template <int NW>
+__global__ void __launch_bounds__(256) batch_sorted_write_kernel(tree_ptrs tp, batch_job* job, uint32_t which) {
+  if (ld32_coherent(&job->bad)) return;
+  if (job->lend) sorted_writes<NW, true>(tp, job, which);
+  else sorted_writes<NW, false>(tp, job, which);
 }
 
 // 9. Finds, each at its batch's snapshot (no writer runs). T: read tile

@@ -1445,14 +1445,15 @@ struct tree_view : tree_ptrs {
   // copy allocates or retires here (kNone: none was reserved, and the tile
   // allocates if the leaf needs it). The leader lane of a leaf whose copy went
   // there gets kTaken.
-  // PLANNED also takes no leaf locks:
-  // in the sorted form's write pass every leaf has one writing tile (the one
-  // that owns its group of sorted writes; a split's new right node holds
-  // only keys of that group) and no reader runs, while the per-key path and
-  // the parents it updates still lock as everywhere else.
-  template <int OP, bool PLANNED = false>
+  // Without LOCK (PLANNED only) no leaf is locked: in the sorted form's write
+  // pass every leaf has one writing tile (the one that owns its group of sorted
+  // writes; a split's new right node holds only keys of that group), so the
+  // locks only serve latest reads (MVBT_CONCURRENT) on other streams. The
+  // per-key path and the parents it updates lock as everywhere else.
+  template <int OP, bool PLANNED = false, bool LOCK = true>
   MVBT_DEV uint64_t write_chunk_at(uint32_t key, uint32_t value, uint64_t q, uint32_t leaf, uint32_t cur,
                                    uint32_t& result, write_ctx& c, const tile_t& t, uint32_t& planned) const {
+    static_assert(PLANNED || LOCK, "see above");
     constexpr int LB = kLeafBatch;
     if constexpr (NW > 32) {
       return q;  // 64-pair nodes: register budget; per-key path
@@ -1472,7 +1473,7 @@ struct tree_view : tree_ptrs {
       }
       // 1. lock every leaf of the chunk at once (each leader lane its own leaf)
       uint32_t old = kLockBit;
-      if (PLANNED) old = 0;  // see above: these leaves have no other writer
+      if (!LOCK) old = 0;
       else if ((lead >> r) & 1) old = atomic_or32(lock_word(leaf), kLockBit);
       const uint64_t locked = lead & t.ballot(!(old & kLockBit));
       for (uint64_t m = lead & ~locked; m; m &= m - 1)
@@ -1495,7 +1496,7 @@ struct tree_view : tree_ptrs {
         // are complete: that wait also covers the reloads just issued. A
         // plain store does it: while the word is locked nobody changes it.
         order_release();
-        if (!PLANNED && ((prev >> r) & 1)) st32_coherent(lock_word(leaf), open);
+        if (LOCK && ((prev >> r) & 1)) st32_coherent(lock_word(leaf), open);
         if (!got) break;
         // 3. apply each leaf's keys in registers; a leaf whose keys do not all
         // fit (or that no longer covers one of them) goes per key. 4. The
@@ -1510,7 +1511,7 @@ struct tree_view : tree_ptrs {
           node_t o, n;
           o.p = n.p = img[i];
           const uint64_t meta = o.meta(t);
-          if (!PLANNED && r == l) open = hi32(meta) & ~kLockBit;
+          if (LOCK && r == l) open = hi32(meta) & ~kLockBit;
           const uint64_t mem = todo & t.ballot(my_lead == l);
           bool good = node_t::is_leaf(meta);
           bool chg = false;

@@ -217,3 +217,71 @@ def test_few_operations_in_many_batches(dev, spare, graph):
     st = tree.memory_stats()
     assert st.live_nodes == live and st.reclaimed_nodes == st.retired_total
     assert tree.validate_tree_structure()[0] == ref.size()
+
+
+@pytest.mark.parametrize("nw", [16, 32, 64])
+@pytest.mark.parametrize("nb", [3, 4500])
+def test_latest_reads_beside_small_calls(dev, nw, nb):
+    """MVBT_CONCURRENT reads of the latest version on one stream while small
+    calls run on another: leaves are written under their locks, so keys that no
+    call writes read exactly, written ones as before or after some call, ranges
+    stay sorted, and no leaf is left locked."""
+    import torch
+    rng = np.random.default_rng(nw + nb)
+    init = np.sort(wl.unique_keys(rng, 60_000))
+    vals = wl.value_of(init) & np.uint32(0x3FFFFFFF)
+    still, moved = init[::2], init[1::2]
+    tree = mv.GpuVersionedBTree(pool_nodes=1 << 20, node_width=nw)
+    tree.bulk_build(to_dev(init, dev), to_dev(vals, dev))
+    calls = []
+    for k in range(24):  # updates (values of bit 31), erases and inserts of the moving keys, in turn
+        n = 9000
+        ops = np.zeros((n, 4), np.uint32)
+        ops[:, 1] = rng.choice(moved, size=n, replace=False)
+        ops[:, 0] = rng.choice([mv.OP_INSERT, mv.OP_ERASE], size=n, p=[0.7, 0.3])
+        ops[:, 2] = ops[:, 1] | np.uint32(0x80000000)
+        offs = np.concatenate([[0], np.sort(rng.integers(0, n + 1, size=nb - 1)), [n]]).astype(np.uint64)
+        calls.append((to_dev(ops, dev), to_dev(offs, dev), torch.empty(n, dtype=torch.int32, device=dev)))
+    q = rng.permutation(init)
+    lo = rng.choice(init, size=4000)
+    hi = np.minimum(lo.astype(np.uint64) + wl.span_for(40, init.size), 0xFFFFFFFE).astype(np.uint32)
+    L = 128
+    dq, dlo, dhi = to_dev(q, dev), to_dev(lo, dev), to_dev(hi, dev)
+    tree.reserve_batches(9000, nb)
+    torch.cuda.synchronize()
+    sr, sw = torch.cuda.Stream(), torch.cuda.Stream()
+    finds, ranges = [], []
+    for ops, offs, res in calls:
+        with torch.cuda.stream(sw):
+            tree.run_batches(ops, offs, results=res, stream=sw)
+        with torch.cuda.stream(sr):
+            finds.append(tree.find(dq, stream=sr, concurrent=True))
+            ranges.append(tree.range_query(dlo, dhi, L, stream=sr, concurrent=True))
+    torch.cuda.synchronize()
+    assert tree.error_flags() == 0
+    unmoved = np.isin(q, still)
+    want = vals[np.searchsorted(init, q)]
+    for f in finds:
+        got = to_np(f)
+        assert np.array_equal(got[unmoved], want[unmoved])
+        m = ~unmoved
+        assert np.all((got[m] == want[m]) | (got[m] == (q[m] | np.uint32(0x80000000))) | (got[m] == 0xFFFFFFFF))
+    a, b = np.searchsorted(still, lo), np.searchsorted(still, hi)
+    for p, c in ranges:
+        p, c = to_np(p, np.uint64).reshape(-1, L), to_np(c)
+        assert c.max() <= L
+        for i in range(0, lo.size, 37):
+            k = (p[i, :c[i]] & np.uint64(0xFFFFFFFF)).astype(np.uint32)
+            assert np.all(np.diff(k.astype(np.int64)) > 0)
+            assert np.array_equal(k[np.isin(k, still)], still[a[i]:b[i]])
+    state = dict(zip(init.tolist(), vals.tolist()))
+    for ops, _, _ in calls:
+        o = to_np(ops).reshape(-1, 4)
+        for ty, k, v in zip(o[:, 0].tolist(), o[:, 1].tolist(), o[:, 2].tolist()):
+            if ty == mv.OP_INSERT:
+                state[k] = v
+            else:
+                state.pop(k, None)
+    assert tree.validate_tree_structure()[0] == len(state)  # (a locked leaf fails this)
+    got = to_np(tree.find(dq))
+    assert np.array_equal(got, np.array([state.get(k, 0xFFFFFFFF) for k in q.tolist()], np.uint32))
