@@ -60,7 +60,6 @@ struct alignas(128) batch_job {
   uint32_t* results;     // one word per op
   uint64_t* pairs;       // range output
   unsigned long long pair_slots;  // capacity of `pairs` in slots of L pairs
-  uint32_t* base_out;    // optional: receives clock0
   uint32_t clock0;
   uint32_t hash_mask;    // conflict table size - 1: a power of two >= 2 * writes (batch_mask_kernel)
   unsigned long long first_op;  // offsets[0]
@@ -140,7 +139,6 @@ __global__ void batch_setup_kernel(batch_job* job, tree_state* st, batch_params 
   job->results = p.results;
   job->pairs = p.pairs;
   job->pair_slots = p.pair_slots;
-  job->base_out = p.base_out;
   job->clock0 = __hip_atomic_fetch_add(&st->clock, p.nb, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
   job->hash_cap_mask = p.hash_mask;
   job->hash_mask = 1023u;

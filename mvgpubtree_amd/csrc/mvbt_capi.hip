@@ -786,8 +786,6 @@ uint32_t worker_blocks(const mvbt_tree* t) {
   return (uint32_t)std::max<uint64_t>(b, 1);
 }
 
-uint32_t worker_blocks(const mvbt_tree* t);
-
 // The sorted form's launch sequence after setup/clear/count: enqueued on a
 // stream, or added to a graph, through `add(fn, grid, block, args)`.
 // Radix passes cover the bits of the largest sort key (the pool capacity).
