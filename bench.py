@@ -578,7 +578,7 @@ def batched_vs_plain(w, L, dev, nw: int, mode: int, waves: int, plain: bool = Tr
 def run_config4(args):
     """Batched form (config 4): 4096 batches, sizes log-uniform in [32, 65536],
     mix 60/20/10/10 find/insert/erase/range (8-128 keys), on a 40M-key tree.
-    The persistent work-queue launch (captured hipGraph, autotuned node width,
+    The batched form in one call (captured hipGraph, autotuned node width,
     worker mode and waves/CU) against the plain per-batch launch path on an
     identical tree."""
     import torch

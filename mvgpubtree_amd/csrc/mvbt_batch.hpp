@@ -1,12 +1,19 @@
-// Persistent work-queue form: many batches of mixed operations in one launch.
+// Batched form: many batches of mixed operations in one call.
 //
 // Semantics (identical to issuing the batches one by one through the plain
 // per-batch API with a snapshot before each): batch b reads (find, range) at
 // snapshot clock0 + b, i.e. it sees exactly the writes of batches < b; its
-// writes (insert, erase) are stamped clock0 + b + 1. The launch reserves the
+// writes (insert, erase) are stamped clock0 + b + 1. The call reserves the
 // nb snapshot ids by advancing the tree clock by nb.
 //
-// Scheduling: tiles claim operations one at a time from one queue, in order
+// Two forms. The sorted form (worker modes 2 and 3; calls of up to kSmallOps
+// operations in fewer launches) applies all writes of a window of batches first,
+// leaf by leaf in batch order, then answers all its reads at their snapshots; it
+// is described from batch_slice_kernel on. The persistent worker (modes 0 and 1,
+// which only the autotuner and callers that ask for them use) works through one
+// queue of the call's operations:
+//
+// Scheduling: tiles claim operations one at a time from the queue, in order
 // (see the worker). An operation of batch b may run once every write of batches < b has
 // completed (a device frontier F = last batch whose writes are all done). A
 // write of batch b must also wait for that, because leaf version chains are
@@ -17,9 +24,9 @@
 // spins inside a branch (the tiles of a wave run in lockstep).
 //
 // A batch's writes must name distinct keys: two writes of one key inside a
-// batch would make the result depend on which tile runs first. The count
-// pass checks this with a hash table over (batch, key) of the call's write
-// operations and rejects the whole call (kErrBadBatch; nothing is applied,
+// batch would make the result depend on which tile runs first. Both forms
+// check this with a hash table over (batch, key) of the call's write
+// operations and reject the whole call (kErrBadBatch; nothing is applied,
 // results are left as they were) when a key repeats, an operation type is
 // unknown, or the offsets disagree with the operation count.
 //
@@ -51,7 +58,7 @@ struct alignas(16) write_rec {
 };
 
 struct alignas(128) batch_job {
-  // per-call parameters (written by batch_setup_kernel)
+  // per-call parameters (written by batch_setup_kernel or batch_small_begin_kernel)
   const op_record* ops;
   unsigned long long nops;  // one past the last op index (= offsets[nb])
   const unsigned long long* offsets;  // nb + 1 absolute op indices into ops
@@ -82,11 +89,13 @@ struct alignas(128) batch_job {
   // operation unless stated.
   uint32_t* list;        // the call's finds, then its ranges (index - first_op), in operation order
   write_rec* writes;     // the call's writes, in operation order
-  uint32_t* w_par;       // parent hint of each write of the window
+  uint32_t* w_par;       // parent hint of each write of the window; after the gather the lent
+                         // slots (lend_slots)
   uint32_t* sort_k[2];   // leaf hints (sort keys), two buffers; the spare one then holds the
                          // sorted writes' parent hints
   uint32_t* sort_v[2];   // positions in the window's writes (sort payloads), two buffers; the
-                         // spare one then holds the sorted writes' copy slots
+                         // spare one then holds the sorted writes' copy slots (lent: and the first
+                         // one their groups)
   write_rec* sorted;     // the window's writes in sorted order
   uint32_t* seg;         // segment counts: kOpClasses * kSliceWaves
   uint32_t* hist;        // kRadix * kSortSegments histogram + kRadix digit totals
@@ -1081,11 +1090,12 @@ __global__ void __launch_bounds__(kSortBlock) batch_assign_kernel(batch_job* job
 
 // ---- small calls of the sorted form ----------------------------------------
 // A call of at most kSmallOps operations in at most kSmallBatches batches: a
-// launch costs 4-5 us whatever it does, and the 24 of a window are most of such
-// a call (3000 operations: 146 us on the batch-after-batch worker, no less in
-// the launches above). One workgroup therefore does the checks and the split,
-// and after the routing one workgroup sorts the writes in LDS and plans their
-// copies: the call is 8 launches.
+// launch costs 4-5 us whatever it does, and the launches above, 13 and 3 more a
+// radix pass, are most of such a call (3 batches of 3000 operations: no less than
+// the 146 us of the batch-after-batch worker). One workgroup therefore does the
+// checks and the split, and after the routing one workgroup sorts the writes in
+// LDS and plans their copies: the call is 7 launches (89 us), besides the
+// maintenance launch that a call after another write begins with.
 constexpr uint32_t kSmallOps = 16384, kSmallBatches = 4096, kSmallBlock = 1024;
 
 // Exclusive prefix of `v` over the workgroup's threads; *total: its sum. `w`:
@@ -1242,8 +1252,9 @@ __global__ void __launch_bounds__(kSmallBlock) batch_small_begin_kernel(batch_jo
 }
 
 // S2. Sort by leaf, gather and copy planning of a small call's writes, by one
-// workgroup: three 8-bit radix passes (bits covers the pool's indices) with
-// leaf and position in LDS, each wave ranking its own stretch; then the gather
+// workgroup: an 8-bit radix pass for every eight bits of the pool's size (three
+// below 2^24 nodes) with leaf and position in LDS, each wave ranking its own
+// stretch; then the gather
 // and the groups as in batch_gather_kernel. The sorted leaf hints end in
 // sort_k[1], as after an odd number of passes.
 __global__ void __launch_bounds__(kSmallBlock) batch_small_plan_kernel(batch_job* job, tree_ptrs tp, uint32_t bits) {

@@ -786,8 +786,8 @@ uint32_t worker_blocks(const mvbt_tree* t) {
   return (uint32_t)std::max<uint64_t>(b, 1);
 }
 
-// The sorted form's launch sequence after setup/clear/count: enqueued on a
-// stream, or added to a graph, through `add(fn, grid, block, args)`.
+// The sorted form's launch sequences (below) are enqueued on a stream, or added
+// to a graph, through `add(fn, grid, block, args)`.
 // Radix passes cover the bits of the largest sort key (the pool capacity).
 uint32_t sort_passes(const mvbt_tree* t) {
   const uint32_t cap = (uint32_t)t->cfg.pool_nodes;
@@ -951,9 +951,10 @@ uint32_t graph_index(const mvbt_tree* t, uint32_t windows) {
 
 // The form of a call. Modes 2 and 3 both run the sorted form, small calls of one
 // window in the form made for them. Mode 3 once ran calls below kAutoSortedOps
-// operations on the persistent worker, whose batches wait for each other: 146 us
-// for 3 batches of 3000 operations against 93 now, 422 against 145 for 24 of
-// 16384. Such calls still keep their version copies until mvbt_reclaim.
+// operations on the persistent worker, whose batches wait for each other: with a
+// reclamation after each call, 245 us for 3 batches of 3000 operations against
+// 120, 546 against 152 for 24 of 682. Such calls still keep their version copies
+// until mvbt_reclaim, in slots lent to them (lend_slots).
 constexpr uint64_t kAutoSortedOps = 16384;
 bool keeps_copies(const mvbt_tree* t, uint64_t num_ops) { return t->worker_mode == 3 && num_ops < kAutoSortedOps; }
 bool small_call(const mvbt_tree* t, uint64_t num_ops, uint32_t num_batches) {

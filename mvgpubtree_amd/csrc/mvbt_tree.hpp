@@ -978,8 +978,8 @@ struct tree_view : tree_ptrs {
         // An entry whose pivot is <= key (entry 0 routes from the node's low
         // bound), by halving steps: the last one in a whole image. In a torn
         // one entry l still has a pivot <= key (or is entry 0), so its child
-        // lies at or left of the right one. Five dependent LDS reads a level
-        // instead of 29 that the LDS serves one wave after another.
+        // lies at or left of the right one. log2(NW) dependent LDS reads a level
+        // instead of one an entry, which the LDS serves one wave after another.
         uint32_t l = 0;
 #pragma unroll
         for (uint32_t step = NW / 2; step != 0; step >>= 1) {

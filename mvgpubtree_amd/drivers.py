@@ -6,9 +6,9 @@
   reference's host API). The loop runs in C++ over the C ABI
   (``libmvbt_driver.so``, csrc/per_batch_driver.cpp), so the comparison with
   the batched form measures device paths, not an interpreter's loop.
-* ``BatchedRunner`` - the persistent work-queue form: the whole stream of
-  batches in one ``run_batches`` launch, optionally through the captured
-  hipGraph.
+* ``BatchedRunner`` - the batched form: the whole stream of batches in one
+  ``run_batches`` call (the sorted form, unless the tree's worker mode names the
+  persistent worker), optionally through the captured hipGraph.
 
 Both produce the same observable results for the same batches.
 """
@@ -137,7 +137,7 @@ class PerBatchRunner:
 
 
 class BatchedRunner:
-    """Device-resident op stream for the persistent form."""
+    """Device-resident op stream for the batched form."""
 
     def __init__(self, batches, L: int, dev, seed: int = 0):
         import torch
